@@ -318,11 +318,12 @@ int lyap_timing_collect(lyap_ctx *ctx, double *kernel_ms, uint64_t *launches)
 int lyap_last_evals(lyap_ctx *ctx, uint64_t *count)
 {
     if (!ctx || !count) return LYAP_ERR_INVALID_ARGUMENT;
-    unsigned long long c = 0;
-    const uint32_t *src = ctx->last_counters ? ctx->last_counters : ctx->counters;
-    LYAP_HIP(ctx, hipMemcpyAsync(&c, src + 2, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
+    *count = 0;
+    if (!ctx->last_counters) return LYAP_OK;
+    std::vector<uint64_t> words(kEvalSlots * kEvalStride);
+    LYAP_HIP(ctx, hipMemcpyAsync(words.data(), ctx->last_counters, kEvalBytes, hipMemcpyDeviceToHost, ctx->stream));
     LYAP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *count = c;
+    *count = sum_evals(words.data());
     return LYAP_OK;
 }
 

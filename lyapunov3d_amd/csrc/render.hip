@@ -939,6 +939,14 @@ __device__ __forceinline__ uint32_t uniform(uint32_t x)
     return __builtin_amdgcn_readfirstlane(x);
 }
 
+/* Adds the lanes' evaluation counts to the wave's slot of the launch's count
+ * (one atomic per wave). */
+__device__ __forceinline__ void count_evals(unsigned long long *counter, unsigned long long n, uint32_t wid)
+{
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off);
+    if (__lane_id() == 0 && n) atomicAdd(counter + wid % kEvalSlots * kEvalStride, n);
+}
+
 /* The chunks of up to 64 lists, held across a wave: lane j holds list j's
  * entry count and the chunks of lists 0..j (an inclusive scan), so a chunk
  * finds its list with one ballot. The counts come in one vector load rather
@@ -1547,10 +1555,7 @@ void render_persistent(const ViewDesc *__restrict__ views, RenderArgs a)
         }
     }
     if (sh_count) shade_list(views[uniform(cur_view)], sh, sh_count);
-    /* one 64-bit atomic per wave for the evaluation count */
-    unsigned long long sum = done_evals;
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off);
-    if (lane == 0 && sum) atomicAdd(a.eval_counter, sum);
+    count_evals(a.eval_counter, done_evals, wid);
     if (a.wave_log && lane == 0 && wid < 8192u) {
         unsigned long long *o = a.wave_log + kWaveLogWords * (wid + 8192ull * a.level);
         o[0] = rounds;
@@ -1663,11 +1668,11 @@ __device__ __forceinline__ uint32_t cont_count(const ViewDesc *__restrict__ view
  * sub-lists hold all its rays together, and a full sub-list has every one of
  * its slots written, so each ray finds a slot within kContSubs tries. */
 __device__ __forceinline__ void append_cont(const ViewDesc &v, uint32_t vi, const Ray &r, bool want,
-                                            PassRec *out, uint32_t *counts)
+                                            PassRec *out, uint32_t *counts, uint32_t first = 0)
 {
     const uint32_t lane = __lane_id();
     const uint32_t sub_cap = v.cont_cap / kContSubs;
-    for (uint32_t tries = 0; tries < kContSubs && __ballot(want) != 0; ++tries) {
+    for (uint32_t tries = first; tries < kContSubs && __ballot(want) != 0; ++tries) {
         const uint64_t m = __ballot(want);
         const uint32_t sub = (blockIdx.x + tries) % kContSubs;
         uint32_t base = 0;
@@ -1683,6 +1688,116 @@ __device__ __forceinline__ void append_cont(const ViewDesc &v, uint32_t vi, cons
             }
         }
     }
+}
+
+/* Parks the rays of this wave's lanes with `want` (leaders) in view vi's
+ * refinement records: the sub-region of this block's XCD, the next ones while
+ * a sub-region is full (the regions hold twice the view's rays, so one has
+ * room). One atomic per wave and try. */
+__device__ __forceinline__ RefineRec refine_record(const Ray &r)
+{
+    RefineRec q;
+    q.pix = r.pix;
+    q.evals = r.evals;
+    q.Vx = r.V.x;
+    q.Vy = r.V.y;
+    q.Vz = r.V.z;
+    q.lo = r.lo();
+    q.hi = r.hi();
+    q.l_hi = r.l_hi();
+    q.dt = r.dt;
+    q.a = r.a;
+    q.c = r.c;
+    q.l_lo = r.l_lo();
+    return q;
+}
+
+__device__ __forceinline__ void append_refine(const ViewDesc &v, uint32_t vi, const Ray &r, bool want,
+                                              RefineRec *out, uint32_t *counts, uint32_t first = 0)
+{
+    const uint32_t lane = __lane_id();
+    for (uint32_t tries = first; tries < kRefineSubs && __ballot(want) != 0; ++tries) {
+        const uint64_t m = __ballot(want);
+        const uint32_t sub = (blockIdx.x + tries) % kRefineSubs;
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(counts + (vi * kRefineSubs + sub) * kHeadStride, (uint32_t)__popcll(m));
+        base = uniform((uint32_t)__shfl((int)base, 0));
+        if (want) {
+            const uint32_t slot = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            if (slot < v.refine_cap) {
+                out[v.refine_base + sub * v.refine_cap + slot] = refine_record(r);
+                want = false;
+            }
+        }
+    }
+}
+
+/* A block's four waves append together: device-scope atomics on one address
+ * take about 20 ns each, one after the other, and the 10,000 waves of a
+ * 512 x 512 frame's first pass share eight addresses (39 us with an atomic
+ * per wave and list, 34 us with one per block). Per wave the view and the
+ * rays to list and to park; the first wave of each view present takes the
+ * reservations for all of that view's waves. */
+struct BlockAppend {
+    uint32_t view[4], n_cont[4], n_refine[4];
+    uint32_t cont_base[4], refine_base[4];
+};
+
+/* Every wave of the block calls this (a wave without rays with no bits in
+ * either mask). Rays that do not fit go on to the next sub-lists. */
+__device__ __forceinline__ void append_block(BlockAppend &s, const ViewDesc &v, uint32_t vi, const Ray &r,
+                                             bool cont, bool park, const PassArgs &a)
+{
+    const uint32_t lane = __lane_id();
+    const uint32_t w = threadIdx.x >> 6;
+    const uint64_t cm = __ballot(cont), pm = __ballot(park);
+    if (lane == 0) {
+        s.view[w] = vi;
+        s.n_cont[w] = (uint32_t)__popcll(cm);
+        s.n_refine[w] = (uint32_t)__popcll(pm);
+    }
+    __syncthreads();
+    /* lane 0 of a view's first wave reserves list entries, lane 1 records */
+    uint32_t first = w, before_c = 0, before_p = 0, total_c = 0, total_p = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        if (s.view[k] != vi) continue;
+        if (k < first) first = k;
+        if (k < w) {
+            before_c += s.n_cont[k];
+            before_p += s.n_refine[k];
+        }
+        total_c += s.n_cont[k];
+        total_p += s.n_refine[k];
+    }
+    if (w == first) {
+        if (lane == 0 && total_c)
+            s.cont_base[w] = atomicAdd(a.out_counts + (vi * kContSubs + blockIdx.x % kContSubs) * kHeadStride, total_c);
+        if (lane == 1 && total_p)
+            s.refine_base[w] =
+                atomicAdd(a.refine_counts + (vi * kRefineSubs + blockIdx.x % kRefineSubs) * kHeadStride, total_p);
+    }
+    __syncthreads();
+    const uint64_t below = (1ull << lane) - 1ull;
+    if (cont) {
+        const uint32_t sub_cap = v.cont_cap / kContSubs;
+        const uint32_t slot = s.cont_base[first] + before_c + (uint32_t)__popcll(cm & below);
+        if (slot < sub_cap) {
+            PassRec q;
+            store_pass(r, q);
+            a.cont_out[v.cont_base + (blockIdx.x % kContSubs) * sub_cap + slot] = q;
+            cont = false;
+        }
+    }
+    if (park) {
+        const uint32_t slot = s.refine_base[first] + before_p + (uint32_t)__popcll(pm & below);
+        if (slot < v.refine_cap) {
+            a.refine_out[v.refine_base + (blockIdx.x % kRefineSubs) * v.refine_cap + slot] = refine_record(r);
+            park = false;
+        }
+    }
+    append_cont(v, vi, r, cont, a.cont_out, a.out_counts, 1u);
+    append_refine(v, vi, r, park, a.refine_out, a.refine_counts, 1u);
 }
 
 /* Every pixel ray of every view, one lane each (a block's 256 rays belong
@@ -1752,6 +1867,7 @@ template <int W, int PREC, bool DRAIN>
 __global__ __launch_bounds__(256) void march_pass(const ViewDesc *__restrict__ views, PassArgs a)
 {
     __shared__ PassStash stash[4];
+    __shared__ BlockAppend appends;
     PassStash &st = stash[threadIdx.x >> 6];
     const uint32_t lane = __lane_id();
     const uint32_t K = uniform(a.K);
@@ -1775,9 +1891,14 @@ __global__ __launch_bounds__(256) void march_pass(const ViewDesc *__restrict__ v
             chunks += (cont_count(views, a.in_counts, p / kContSubs, p % kContSubs) + per - 1u) / per;
     }
     uint32_t done_evals = 0;
-    for (uint32_t c = wid; c < chunks; c += n_waves) {
+    /* the four waves of a block take neighbouring chunks; the one-round
+     * passes append as a block, so a wave past the last chunk stays (without
+     * rays) while others of its block have one */
+    for (uint32_t c = wid; (DRAIN ? c : c - (wid & 3u)) < chunks; c += n_waves) {
         uint32_t acc = 0, p = 0, cnt = 0;
-        if (held) {
+        if (!DRAIN && c >= chunks) {
+            acc = c;
+        } else if (held) {
             chunk_find(cm, c, per, p, acc, cnt);
         } else {
             for (; p < pairs; ++p) {
@@ -1833,47 +1954,18 @@ __global__ __launch_bounds__(256) void march_pass(const ViewDesc *__restrict__ v
             combine_march<PassStash, 64u>(v, r, evm, st, gbase, K, busy ? (int)PH_MARCH : (int)PH_IDLE,
                                           rank == 0, finished);
             if (finished && rank == 0) done_evals += r.evals;
-            /* park the rays that found their opaque sample: sub-region by
-             * block, the next ones while a sub-region is full (the regions
-             * hold twice the view's rays, so one has room) */
-            bool pk = busy && rank == 0 && r.phase == PH_REFINE;
-            for (uint32_t tries = 0; tries < kRefineSubs && __ballot(pk) != 0; ++tries) {
-                const uint64_t pm = __ballot(pk);
-                const uint32_t sub = (blockIdx.x + tries) % kRefineSubs;
-                uint32_t base = 0;
-                if (lane == 0)
-                    base = atomicAdd(a.refine_counts + (vi * kRefineSubs + sub) * kHeadStride,
-                                     (uint32_t)__popcll(pm));
-                base = uniform((uint32_t)__shfl((int)base, 0));
-                if (pk) {
-                    const uint32_t slot = base + (uint32_t)__popcll(pm & ((1ull << lane) - 1ull));
-                    if (slot < v.refine_cap) {
-                        RefineRec q;
-                        q.pix = r.pix;
-                        q.evals = r.evals;
-                        q.Vx = r.V.x;
-                        q.Vy = r.V.y;
-                        q.Vz = r.V.z;
-                        q.lo = r.lo();
-                        q.hi = r.hi();
-                        q.l_hi = r.l_hi();
-                        q.dt = r.dt;
-                        q.a = r.a;
-                        q.c = r.c;
-                        q.l_lo = r.l_lo();
-                        a.refine_out[v.refine_base + sub * v.refine_cap + slot] = q;
-                        pk = false;
-                    }
-                }
-            }
+            const bool park = busy && rank == 0 && r.phase == PH_REFINE;
             busy = busy && r.phase == PH_MARCH;
-            if (!DRAIN || (a.rounds != 0 && round + 1u >= a.rounds) || __ballot(busy) == 0) break;
+            if (!DRAIN) {
+                append_block(appends, v, vi, r, busy && rank == 0, park, a);
+                break;
+            }
+            append_refine(v, vi, r, park, a.refine_out, a.refine_counts);
+            if ((a.rounds != 0 && round + 1u >= a.rounds) || __ballot(busy) == 0) break;
         }
-        append_cont(v, vi, r, busy && rank == 0, a.cont_out, a.out_counts);
+        if (DRAIN) append_cont(v, vi, r, busy && rank == 0, a.cont_out, a.out_counts);
     }
-    unsigned long long sum = done_evals;
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off);
-    if (lane == 0 && sum) atomicAdd(a.eval_counter, sum);
+    count_evals(a.eval_counter, done_evals, wid);
 }
 
 /* ---- refinement launch -------------------------------------------------- */
@@ -2019,8 +2111,7 @@ __global__ __launch_bounds__(256) void refine_rays(const ViewDesc *__restrict__ 
             done += evals + 6u;
         }
     }
-    for (int off = 32; off > 0; off >>= 1) done += __shfl_down(done, off);
-    if (lane == 0 && done) atomicAdd(a.eval_counter, done);
+    count_evals(a.eval_counter, done, wid);
 }
 /* ---- FP64 pass over the volume blocks' lists ---------------------------- */
 
@@ -2263,9 +2354,10 @@ static LaunchPlan plan_launch(const lyap_ctx *ctx, uint64_t rays, const LyapTuni
 /* Device and pinned memory one launch sequence uses. The context owns one
  * set for its direct calls; a captured frame owns its own, so a replay never
  * sees memory that a later call reallocated. */
-/* Words of the counter block: the evaluation count in the first cache line,
- * then kTileHeads claim counters per launch level. */
-constexpr uint32_t kCounterWords = kHeadStride + 4u * kTileHeads * kHeadStride;
+/* Words of the counter block: the evaluation counts, then kTileHeads claim
+ * counters per launch level. */
+constexpr uint32_t kEvalWords = (uint32_t)(kEvalBytes / sizeof(uint32_t));
+constexpr uint32_t kCounterWords = kEvalWords + 4u * kTileHeads * kHeadStride;
 
 struct RenderResources {
     void *view_table = nullptr;      /* device ViewDesc[] */
@@ -2277,7 +2369,7 @@ struct RenderResources {
     size_t staging_bytes[2] = {0, 0};
     hipEvent_t staged[2] = {nullptr, nullptr};
     uint32_t stage = 0;              /* staging buffer of the latest launch */
-    uint32_t *counters = nullptr;    /* kCounterWords: [2..3] evaluations, then tile heads */
+    uint32_t *counters = nullptr;    /* kCounterWords: evaluation counts, then tile heads */
     void *cont_buf = nullptr;        /* rays handed between levels */
     size_t cont_buf_bytes = 0;
     void *cont_counts = nullptr;     /* per view and level */
@@ -2490,7 +2582,7 @@ static int launch_refine(lyap_ctx *ctx, const RenderResources &res, unsigned n_v
     ra.n_views = n_views;
     ra.recs = (const RefineRec *)res.refine_buf;
     ra.counts = (const uint32_t *)res.refine_counts;
-    ra.eval_counter = (unsigned long long *)(res.counters + 2);
+    ra.eval_counter = (unsigned long long *)res.counters;
     const uint32_t cus = ctx->num_cus > 0 ? (uint32_t)ctx->num_cus : 256u;
     const uint32_t blocks = cus * 8u;
 #define LYAP_LAUNCH(WW, PP, MM)                                                                     \
@@ -2547,7 +2639,7 @@ static int enqueue_passes(lyap_ctx *ctx, RenderResources &res, const ViewDesc *v
     a.n_views = n_views;
     a.refine_out = (RefineRec *)res.refine_buf;
     a.refine_counts = (uint32_t *)res.refine_counts;
-    a.eval_counter = (unsigned long long *)(res.counters + 2);
+    a.eval_counter = (unsigned long long *)res.counters;
     a.cont_out = buf[0];
     a.out_counts = counts;
     int rc = timing_mark(ctx);
@@ -2657,8 +2749,8 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
         a.tile_rays = plan.tile_rays;
         a.lanes_per_ray = plan.lanes_per_ray;
         a.slots = plan.slots;
-        a.tile_heads = res.counters + kHeadStride + level * kTileHeads * kHeadStride;
-        a.eval_counter = (unsigned long long *)(res.counters + 2);
+        a.tile_heads = res.counters + kEvalWords + level * kTileHeads * kHeadStride;
+        a.eval_counter = (unsigned long long *)res.counters;
         a.wave_log = (unsigned long long *)ctx->debug_wave_log;
         a.level = level;
         a.budget = level_budget(level, plan);

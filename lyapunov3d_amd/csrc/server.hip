@@ -36,7 +36,7 @@ struct HipSlot {
     RenderSlot *rs = nullptr;
     hipEvent_t start = nullptr, end = nullptr;
     /* pinned: the launch's lambda evaluations (rays' samples, one per voxel) */
-    unsigned long long *host_evals = nullptr;
+    uint64_t *host_evals = nullptr;   /* kEvalSlots counts (a volume slot: word 0) */
     /* pinned: FP64 re-evaluations of each slab, kItemCountStride words apart */
     uint32_t *host_reeval = nullptr;
     unsigned nblocks = 0;
@@ -60,11 +60,11 @@ public:
             if (rc) return fail(owner_, rc, "server slot context: %s", lyap_strerror(rc));
             const size_t reeval_bytes = kMaxSlabs * kItemCountStride * sizeof(uint32_t);
             if (hipEventCreate(&sl.start) != hipSuccess || hipEventCreate(&sl.end) != hipSuccess ||
-                hipHostMalloc((void **)&sl.host_evals, sizeof(unsigned long long), hipHostMallocDefault) !=
+                hipHostMalloc((void **)&sl.host_evals, kEvalBytes, hipHostMallocDefault) !=
                     hipSuccess ||
                 hipHostMalloc((void **)&sl.host_reeval, reeval_bytes, hipHostMallocDefault) != hipSuccess)
                 return fail(owner_, LYAP_ERR_DEVICE, "server slot set-up failed");
-            *sl.host_evals = 0;
+            std::memset(sl.host_evals, 0, kEvalBytes);
             std::memset(sl.host_reeval, 0, reeval_bytes);
             if (sl.kind != SLOT_VOLUME) {
                 sl.rs = render_slot_create();
@@ -124,7 +124,7 @@ public:
         if (q != hipSuccess) return fail(owner_, LYAP_ERR_DEVICE, "server launch: %s", hipGetErrorString(q));
         float ms = 0.0f;
         res->ms = hipEventElapsedTime(&ms, sl.start, sl.end) == hipSuccess ? (double)ms : -1.0;
-        res->evals = *sl.host_evals;
+        res->evals = sl.kind == SLOT_VOLUME ? sl.host_evals[0] : sum_evals(sl.host_evals);
         for (unsigned b = 0; b < sl.nblocks && b < kMaxSlabs; ++b)
             res->reeval[b] = sl.host_reeval[b * kItemCountStride];
         return LYAP_OK;
@@ -165,7 +165,7 @@ private:
                                         (unsigned)l.views.size(), l.blocks.data(), (unsigned)l.blocks.size(),
                                         cfg_.vol_mode, cfg_.mode, owner_->tuned);
             if (rc) return rc;
-            LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_evals, render_slot_counters(sl.rs) + 2, 8,
+            LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_evals, render_slot_counters(sl.rs), kEvalBytes,
                                             hipMemcpyDeviceToHost, sl.ctx->stream));
             if (!l.blocks.empty())
                 LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval,
