@@ -229,6 +229,8 @@ typedef struct LyapRenderMode {
  * instead: a set-up launch lists the rays that meet the box, then launches
  * of one round each give every listed ray K lanes (4, 8, 16, 32, then 64
  * samples at once), the last running its rays to the end of their march.
+ * Views refined by the walk with step jitter run one lane per ray from the
+ * first sample to the last (the next step needs the last sample's lambda).
  * LEVELS: BATCHED without the passes (the persistent launches only).
  * DIRECT: the reference's own launch shape (kernel.cu:500-516): one lane
  * per ray for 64 consecutive rays (an 8x8 pixel block), each lane marching

@@ -27,54 +27,9 @@
 #include <cstring>
 #include <vector>
 
-#include "internal.hpp"
+#include "render_common.hpp"
 
 namespace lyap {
-
-/* One view of a render launch, in device memory. */
-struct ViewDesc {
-    EvalDesc e;
-    LyapCam cam;
-    LyapParams prm;
-    uint32_t w, h;
-    uint32_t blocks_x;         /* 8x8 pixel blocks per row */
-    uint32_t n_rays;           /* 64 * blocks, padded past the image edge */
-    uint32_t tile_begin;       /* first tile of this view in the launch */
-    uint32_t n_tiles;
-    LyapRGBA *rgba;
-    LyapPoint *points;
-    float *depth;
-    float *lambda;
-    uint32_t *evals;
-    const LyapLight *lights;
-    uint32_t num_lights;
-    int32_t refine;            /* LYAP_REFINE_* */
-    int32_t bisect_steps;
-    float normal_h;
-    float margin;              /* FP64 re-evaluation margin during bisection */
-    uint32_t max_samples;
-    uint32_t ray_begin;        /* first ray of this launch (a view may be split) */
-    uint32_t cont_base;        /* this view's region of the continuation buffers */
-    uint32_t cont_cap;
-    uint32_t refine_base;      /* this view's region of the refinement records */
-    uint32_t refine_cap;       /* records per sub-region (kRefineSubs of them) */
-    uint32_t ray_base;         /* march passes: first ray of this view in ray_start's grid */
-    /* Items of a launch are views or volume blocks (kItemVolume). A volume
-     * block is z slices [vz0, vz0 + n_rays / (vnx * vny)) of an vnx * vny * vnz
-     * grid over [vlo, vlo + vspan), lambda written to vol_out (slice vz0) in
-     * the x-fastest layout of kernel.cu:525; voxels the FP32 pass is unsure of
-     * go to the block's region of the FP64 list. */
-    uint32_t kind;
-    uint32_t tile_len;         /* rays or voxels per level-0 work-queue tile */
-    float *vol_out;
-    uint32_t vnx, vny, vnz, vz0;
-    float vlo[3], vspan[3];
-    float vmargin, vtau, vband;
-    uint32_t vlist_base, vlist_cap;
-};
-
-constexpr uint32_t kItemView = 0;
-constexpr uint32_t kItemVolume = 1;
 
 /* March state of a ray handed to the next launch (96 bytes; 16-byte
  * aligned, so a record moves in six 16-byte loads or stores). */
@@ -88,28 +43,6 @@ struct alignas(16) ContEntry {
     uint32_t pad[2];
 };
 static_assert(sizeof(ContEntry) == 96, "continuation record size");
-
-/* A ray whose march found its opaque sample, waiting for the refinement
- * launch: the bisection interval [lo, hi] with lambda at both ends, the
- * march step (the normal offset of the reference's method), the march sums
- * and the evaluations so far (48 bytes). */
-struct alignas(16) RefineRec {
-    uint32_t pix, evals;
-    float Vx, Vy, Vz, lo, hi, l_hi, dt, a, c, l_lo;
-};
-static_assert(sizeof(RefineRec) == 48, "refinement record size");
-
-/* Refinement records of a view are kept in kRefineSubs sub-regions, one per
- * block index modulo kRefineSubs, each with its own counter on a 128-byte
- * line: waves of one XCD share a counter, and device-scope atomics on a line
- * that waves of several XCDs update are slow. */
-constexpr uint32_t kRefineSubs = 8;
-
-/* The march passes list their rays the same way: a view's continuation
- * region is kContSubs sub-lists of cont_cap / kContSubs records, one counter
- * per sub-list on its own 128-byte line, taken by block index modulo
- * kContSubs. */
-constexpr uint32_t kContSubs = 8;
 
 struct RenderArgs {
     const ViewDesc *views;
@@ -149,136 +82,6 @@ namespace {
 enum : int { PH_IDLE = 0, PH_MARCH = 1, PH_REFINE = 2, PH_NORMAL = 3 };
 
 constexpr uint32_t kMaxWalk = 64;
-
-struct F3 { float x, y, z; };
-__device__ __forceinline__ F3 f3(const LyapVec &v) { return {v.x, v.y, v.z}; }
-__device__ __forceinline__ F3 add(F3 a, F3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ F3 sub(F3 a, F3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-__device__ __forceinline__ F3 mul(F3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
-__device__ __forceinline__ F3 divv(F3 a, float s) { return {a.x / s, a.y / s, a.z / s}; }
-__device__ __forceinline__ float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ float mag2(F3 a) { return a.x * a.x + a.y * a.y + a.z * a.z; }
-/* Vec::normalize (vec3.hpp:141-154) */
-__device__ __forceinline__ F3 normalized(F3 a)
-{
-    const float m2 = mag2(a);
-    if ((double)m2 < 1e-12) return {0.f, 0.f, 0.f};
-    if (m2 == 1.0f) return a;
-    return divv(a, sqrtf(m2));
-}
-__device__ __forceinline__ float clamp01(float v) { return v < 0.0f ? 0.0f : (v > 1.0f ? 1.0f : v); }
-
-struct C4 { float x, y, z, w; };
-__device__ __forceinline__ C4 col(const LyapColor &c) { return {c.x, c.y, c.z, c.w}; }
-__device__ __forceinline__ C4 cadd(C4 a, C4 b) { return {a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w}; }
-__device__ __forceinline__ C4 cmul(C4 a, float s) { return {a.x * s, a.y * s, a.z * s, a.w * s}; }
-
-/* shade (kernel.cu:25-106) */
-__device__ C4 shade(F3 P, F3 N, float a, float c, const LyapCam &cam,
-                    const LyapLight *lights, uint32_t n_lights)
-{
-    C4 color = {0.f, 0.f, 0.f, 0.f};
-    if (__builtin_isnan(a)) return color;
-    const F3 camC = f3(cam.C);
-    for (uint32_t li = 0; li < n_lights; ++li) {
-        const LyapLight &L = lights[li];
-        const F3 camV = sub(camC, P);
-        F3 lightV = sub(f3(L.C), P);
-        const float d2 = mag2(lightV);
-        lightV = normalized(lightV);
-        float i = dot(lightV, N);
-        const float j = -dot(lightV, f3(L.V));
-        C4 phong;
-        if (j > L.lightOuterCone) {
-            i = clamp01(i);
-            const C4 diffuse = cmul(col(L.diffuseColor), i * L.diffusePower);
-            const F3 halfV = normalized(add(camV, lightV));
-            float s = clamp01(dot(N, halfV));
-            s = powf(s, L.specularHardness);
-            const C4 specular = cmul(col(L.specularColor), s * L.specularPower);
-            phong = cmul(cadd(specular, diffuse), L.lightRange / d2);
-            if (j < L.lightInnerCone)
-                phong = cmul(phong, (j - L.lightOuterCone) / (L.lightInnerCone - L.lightOuterCone));
-            phong = cadd(phong, col(L.ambient));
-        } else {
-            phong = col(L.ambient);
-        }
-        if (c > 0.0f) {
-            const float k = (float)(0.1125 / (double)logf(c));
-            phong = cadd(phong, cmul(col(L.chaosColor), k));
-        }
-        color = cadd(color, phong);
-    }
-    return color;
-}
-
-/* to_rgba (color.hpp:169-175), saturating. */
-__device__ __forceinline__ unsigned char to_u8(float x)
-{
-    const double v = 255.0 * (double)x;
-    if (!(v > 0.0)) return 0;
-    if (v >= 255.0) return 255;
-    return (unsigned char)v;
-}
-
-/* Box entry and exit (kernel.cu:181-285), plane parameters formed in double
- * and stored as float like the reference's double literals make them. */
-__device__ bool clip_box(F3 C, F3 V, float lo, float hi, float &t0_out, float &t1_out)
-{
-    const double dlo = lo, dhi = hi;
-    float ts[6];
-    const float Ca[3] = {C.x, C.y, C.z};
-    const float Va[3] = {V.x, V.y, V.z};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        ts[2 * a] = (Va[a] != 0.0f) ? (float)((dlo - (double)Ca[a]) / (double)Va[a]) : INFINITY;
-        ts[2 * a + 1] = (Va[a] != 0.0f) ? (float)((dhi - (double)Ca[a]) / (double)Va[a]) : INFINITY;
-    }
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        if (ts[k] == INFINITY) continue;
-        const F3 P = add(C, mul(V, ts[k]));
-        const float Pa[3] = {P.x, P.y, P.z};
-        const int ax = k / 2;
-        bool out = false;
-#pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            if (b == ax) continue;
-            if ((double)Pa[b] < dlo || (double)Pa[b] > dhi) out = true;
-        }
-        if (out) ts[k] = NAN;
-    }
-    float t0 = 3.40282347e+38F, t1 = 0.0f;
-    int i0 = -1, i1 = -1;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        if (!__builtin_isfinite(ts[k])) continue;
-        if (i0 == -1 || ts[k] < t0) { t0 = ts[k]; i0 = k; }
-        if (i1 == -1 || ts[k] > t1) { t1 = ts[k]; i1 = k; }
-    }
-    if (i0 == -1 && i1 == -1) return false;
-    if (i1 == -1 || i0 == i1) { t1 = t0; t0 = 0.0f; }
-    if (t0 < 0) t0 = 0.0f;
-    t0_out = t0;
-    t1_out = t1;
-    return true;
-}
-
-/* ---- lambda in the kernel's window ------------------------------------- */
-
-template <int W>
-__device__ __noinline__ float eval_fp64_call(const EvalDesc &e, float x, float y, float z)
-{
-    return (float)lambda_fp64_w<W>(x, y, z, e);
-}
-
-template <int W, int PREC>
-__device__ __forceinline__ float eval_lambda(const EvalDesc &e, float x, float y, float z)
-{
-    if (PREC == LYAP_PREC_FP64) return (float)lambda_fp64_w<W>(x, y, z, e);
-    if (PREC == LYAP_PREC_PLAIN) return lambda_plain_w<W>(x, y, z, e);
-    return lambda_product_w<W>(x, y, z, e);
-}
 
 /* Per-lane ray state. Every lane of a group holds the same copy; the group's
  * lanes differ only in which point they evaluate. */
@@ -355,72 +158,6 @@ __device__ __forceinline__ Ray shuffle_ray(const Ray &r, int src)
     return o;
 }
 
-/* The view's output pointers, read together (one wait for all of them
- * rather than one per optional output). */
-struct OutPtrs {
-    LyapRGBA *rgba;
-    LyapPoint *points;
-    float *depth;
-    float *lambda;
-    uint32_t *evals;
-    uint32_t present;      /* bit 0 points, 1 depth, 2 lambda, 3 evals */
-};
-
-__device__ __forceinline__ OutPtrs out_ptrs(const ViewDesc &v)
-{
-    OutPtrs o;
-    o.rgba = v.rgba;
-    o.points = v.points;
-    o.depth = v.depth;
-    o.lambda = v.lambda;
-    o.evals = v.evals;
-    o.present = (o.points ? 1u : 0u) | (o.depth ? 2u : 0u) | (o.lambda ? 4u : 0u) |
-                (o.evals ? 8u : 0u);
-    return o;
-}
-
-__device__ __forceinline__ void write_miss(const ViewDesc &v, const Ray &r)
-{
-    const OutPtrs o = out_ptrs(v);
-    if (o.present & 1u) {
-        LyapPoint p;
-        p.P = {0.f, 0.f, 0.f};
-        p.N = {0.f, 0.f, 0.f};
-        p.a = NAN;
-        p.c = 0.f;
-        p.l = NAN;
-        o.points[r.pix] = p;
-    }
-    if (o.present & 2u) o.depth[r.pix] = NAN;
-    if (o.present & 4u) o.lambda[r.pix] = NAN;
-    if (o.present & 8u) o.evals[r.pix] = r.evals;
-    LyapRGBA z = {0, 0, 0, 0};
-    o.rgba[r.pix] = z;
-}
-
-/* A NaN normal component (a normal sample's lambda was NaN) as the one
- * quiet NaN: the refinement launch and refinement in place form the
- * differences in orders that agree on every number but not on a NaN's sign
- * bit. */
-__device__ __forceinline__ float canonical(float x) { return __builtin_isnan(x) ? NAN : x; }
-
-__device__ void write_hit(const ViewDesc &v, const Ray &r, F3 N)
-{
-    const OutPtrs o = out_ptrs(v);
-    if (o.present & 1u) {
-        LyapPoint p;
-        p.P = {r.P.x, r.P.y, r.P.z};
-        p.N = {canonical(N.x), canonical(N.y), canonical(N.z)};
-        p.a = r.a;
-        p.c = r.c;
-        p.l = r.l;
-        o.points[r.pix] = p;
-    }
-    if (o.present & 2u) o.depth[r.pix] = r.t;
-    if (o.present & 4u) o.lambda[r.pix] = r.l;
-    if (o.present & 8u) o.evals[r.pix] = r.evals;
-}
-
 /* Hits waiting for their colour, per wave, in LDS. Shading a hit as its
  * ray ends runs the lights loop for one lane of the wave at a time; the
  * wave instead collects up to 64 hits and shades them with all its lanes at
@@ -456,28 +193,6 @@ __device__ void shade_list(const ViewDesc &v, const ShadeList &sl, uint32_t n)
     }
 }
 
-/* Starts ray `id` of view v; returns false (after the leader wrote a miss,
- * or nothing for a padding ray past the image edge) when no evaluation is
- * needed. Every lane of the ray's group runs it and gets the same state. */
-enum : int { RAY_PAD = 0, RAY_MISS = 1, RAY_HIT = 2 };
-
-/* Pixel, direction and box interval of ray `id` of view v (pixel mapping
- * kernel.cu:500-516, direction :160-163, box clip :180-279). RAY_PAD for a
- * padding ray past the image edge. */
-__device__ __forceinline__ int ray_setup(const ViewDesc &v, uint32_t id, uint32_t &pix, F3 &V,
-                                         float &t0, float &t1)
-{
-    id += v.ray_begin;
-    const uint32_t blk = id >> 6, in = id & 63u;
-    const uint32_t px = (blk % v.blocks_x) * 8u + (in & 7u);
-    const uint32_t py = (blk / v.blocks_x) * 8u + (in >> 3);
-    if (px >= v.w || py >= v.h) return RAY_PAD;
-    pix = px + py * v.w;
-    V = add(add(f3(v.cam.S0), mul(f3(v.cam.SDX), (float)px)), mul(f3(v.cam.SDY), (float)py));
-    V = normalized(V);
-    V = divv(V, v.cam.M);
-    return clip_box(f3(v.cam.C), V, v.prm.lMin, v.prm.lMax, t0, t1) ? RAY_HIT : RAY_MISS;
-}
 /* The march state of a ray that meets the box over [t0, t1]
  * (kernel.cu:281-314). Every lane of the ray's group runs it. */
 __device__ __forceinline__ void start_hit(const ViewDesc &v, uint32_t pix, F3 V, float t0,
@@ -707,14 +422,14 @@ __device__ __forceinline__ int march_consume(const ViewDesc &v, Ray &r, float l,
             if (__builtin_isfinite(jit)) step = r.dt * jit;
         }
         if (!march_step(v, r, step)) {
-            if (leader) write_miss(v, r);
+            if (leader) write_miss(v, r.pix, r.evals);
             r.phase = PH_IDLE;
             return 1;
         }
         r.last_step = step;
         ++r.index;
         if (r.t > r.t1 || r.index >= v.max_samples) {
-            if (leader) write_miss(v, r);
+            if (leader) write_miss(v, r.pix, r.evals);
             r.phase = PH_IDLE;
             return 1;
         }
@@ -735,7 +450,6 @@ constexpr uint32_t kMaxSlots = 4;
  * over kTileHeads addresses instead of queueing on one. A block starts on head
  * blockIdx % kTileHeads and moves on when its head runs dry. */
 constexpr uint32_t kTileHeads = 8;
-constexpr uint32_t kHeadStride = 32;          /* 128 bytes */
 constexpr uint32_t kWaveLogWords = 16;
 
 struct RoundStash {
@@ -747,13 +461,6 @@ struct RoundStash {
      * to neither), formed by the lane that evaluated it */
     float ca[64 * kMaxSlots], aa[64 * kMaxSlots];
 };
-
-__device__ __forceinline__ void wave_sync_lds()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 /* The march part of combine: the group's samples j = 0..K-1 (read from the
  * stash at base + j, N entries) were taken at the positions the sequential
@@ -809,7 +516,7 @@ __device__ __forceinline__ void combine_march(const ViewDesc &v, Ray &r, uint64_
             r.P = Pe;
             if (!ve) {
                 /* the step to sample e left the box or could not advance */
-                if (leader) write_miss(v, r);
+                if (leader) write_miss(v, r.pix, r.evals);
                 r.phase = PH_IDLE;
                 finished = true;
             } else {
@@ -821,7 +528,7 @@ __device__ __forceinline__ void combine_march(const ViewDesc &v, Ray &r, uint64_
             r.t = te;
             r.P = Pe;
             if (r.index >= v.max_samples || !march_step(v, r, r.dt) || r.t > r.t1) {
-                if (leader) write_miss(v, r);
+                if (leader) write_miss(v, r.pix, r.evals);
                 r.phase = PH_IDLE;
                 finished = true;
             }
@@ -921,7 +628,7 @@ __device__ bool combine(const ViewDesc &v, Ray &r, uint64_t evm, const RoundStas
         }
         if (ph == PH_NORMAL && r.k >= 6u) {
             const F3 N = normalized({r.gx(), r.gy(), r.gz()});
-            if (leader) write_hit(v, r, N);
+            if (leader) write_hit(v, r.pix, r.evals, r.P, N, r.t, r.l, r.a, r.c);
             /* the colour is computed later, from the normal kept here */
             r.gx() = N.x;
             r.gy() = N.y;
@@ -932,54 +639,6 @@ __device__ bool combine(const ViewDesc &v, Ray &r, uint64_t evm, const RoundStas
         }
     }
     return finished;
-}
-
-__device__ __forceinline__ uint32_t uniform(uint32_t x)
-{
-    return __builtin_amdgcn_readfirstlane(x);
-}
-
-/* Adds the lanes' evaluation counts to the wave's slot of the launch's count
- * (one atomic per wave). */
-__device__ __forceinline__ void count_evals(unsigned long long *counter, unsigned long long n, uint32_t wid)
-{
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off);
-    if (__lane_id() == 0 && n) atomicAdd(counter + wid % kEvalSlots * kEvalStride, n);
-}
-
-/* The chunks of up to 64 lists, held across a wave: lane j holds list j's
- * entry count and the chunks of lists 0..j (an inclusive scan), so a chunk
- * finds its list with one ballot. The counts come in one vector load rather
- * than a walk of dependent scalar loads at every wave's start. */
-struct ChunkMap {
-    uint32_t cnt;      /* lane j: entries of list j (0 past the lists) */
-    uint32_t end;      /* lane j: chunks of lists 0..j */
-    uint32_t total;    /* chunks of all lists */
-};
-
-__device__ __forceinline__ ChunkMap chunk_map(uint32_t cnt, uint32_t per, uint32_t lane)
-{
-    ChunkMap m;
-    m.cnt = cnt;
-    uint32_t x = (cnt + per - 1u) / per;
-#pragma unroll
-    for (uint32_t off = 1; off < 64u; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, off);
-        if (lane >= off) x += y;
-    }
-    m.end = x;
-    m.total = uniform((uint32_t)__shfl((int)x, 63));
-    return m;
-}
-
-/* List p holding chunk c (< m.total), the chunks before p and p's entries.
- * Every lane of the wave takes part. */
-__device__ __forceinline__ void chunk_find(const ChunkMap &m, uint32_t c, uint32_t per, uint32_t &p,
-                                           uint32_t &acc, uint32_t &cnt)
-{
-    p = uniform((uint32_t)__popcll(__ballot(m.end <= c)));
-    cnt = uniform((uint32_t)__shfl((int)m.cnt, (int)p));
-    acc = uniform((uint32_t)__shfl((int)m.end, (int)p)) - (cnt + per - 1u) / per;
 }
 
 /* Rays [first, last) of view `view` for tile t. Level 0 tiles cover the
@@ -1241,10 +900,7 @@ void render_persistent(const ViewDesc *__restrict__ views, RenderArgs a)
                 float t0 = 0.f, t1 = 0.f;
                 const int k = lane < n ? ray_setup(v, pos + lane, pix, V, t0, t1) : RAY_PAD;
                 if (k == RAY_MISS) {
-                    Ray m;
-                    m.pix = pix;
-                    m.evals = 0;
-                    write_miss(v, m);
+                    write_miss(v, pix, 0u);
                 }
                 const uint64_t hits = __ballot(k == RAY_HIT);
                 if (k == RAY_HIT) {
@@ -1328,10 +984,7 @@ void render_persistent(const ViewDesc *__restrict__ views, RenderArgs a)
                     const int k = ray_setup(v, pos + rk, p_pix, p_V, p_t0, p_t1);
                     if (k == RAY_HIT) pend = true;
                     else if (k == RAY_MISS && rank == 0) {
-                        Ray m;
-                        m.pix = p_pix;
-                        m.evals = 0;
-                        write_miss(v, m);
+                        write_miss(v, p_pix, 0u);
                     }
                 } else {
                     p_id = v.cont_base + pos + rk;
@@ -1826,9 +1479,7 @@ __global__ __launch_bounds__(256) void ray_start(const ViewDesc *__restrict__ vi
     Ray r;
     r.phase = PH_IDLE;
     if (k == RAY_MISS) {
-        r.pix = pix;
-        r.evals = 0;
-        write_miss(v, r);
+        write_miss(v, pix, 0u);
     } else if (k == RAY_HIT) {
         start_hit(v, pix, V, t0, t1, r);
     }
@@ -2100,7 +1751,7 @@ __global__ __launch_bounds__(256) void refine_rays(const ViewDesc *__restrict__ 
         if (has && side == 0) {
             r.evals = evals + 6u;
             const F3 N = normalized({g[0], g[1], g[2]});
-            write_hit(v, r, N);
+            write_hit(v, r.pix, r.evals, r.P, N, r.t, r.l, r.a, r.c);
             const C4 cc = shade(r.P, N, r.a, r.c, v.cam, v.lights, v.num_lights);
             LyapRGBA px;
             px.r = to_u8(cc.x);
@@ -2424,6 +2075,17 @@ static bool parks(const LaunchPlan &plan, const ViewDesc *views)
            views[0].bisect_steps > 0;
 }
 
+/* Whether the launch runs in walk_rays: every item a view refined by the
+ * walk whose step jitter keeps its samples from being taken ahead. */
+static bool walks(const LaunchPlan &plan, const ViewDesc *views, unsigned n_views)
+{
+    if (plan.direct || plan.levels) return false;
+    for (unsigned i = 0; i < n_views; ++i)
+        if (views[i].kind != kItemView || views[i].refine != LYAP_REFINE_WALK || views[i].prm.jitter == 0.0f)
+            return false;
+    return n_views > 0;
+}
+
 /* March passes (march_pass): the lanes per ray of each pass, at most
  * kMaxPasses of them; rays still marching after the last pass finish in a
  * persistent launch. */
@@ -2736,6 +2398,15 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
     /* volume blocks finish at level 0; later levels carry rays only */
     uint32_t levels = (plan.direct || !has_rays) ? 1u : 4u;
     uint32_t first_level = 0;
+    if (walks(plan, views, n_views)) {
+        uint64_t rays = 0;
+        for (unsigned i = 0; i < n_views; ++i) rays += (views[i].n_rays + 255u) / 256u * 256u;
+        rc = timing_mark(ctx);
+        if (rc) return rc;
+        rc = launch_walk(ctx, res.view_table, n_views, rays, res.counters, W, precision);
+        if (rc) return rc;
+        return timing_mark(ctx);
+    }
     if (pp.n > 0) {
         /* the passes march every ray to its end: no level launch follows */
         rc = enqueue_passes(ctx, res, views, n_views, pp, W, precision);
