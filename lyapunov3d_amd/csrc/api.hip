@@ -67,10 +67,10 @@ int ensure_reeval_list(lyap_ctx *ctx, size_t entries)
 }
 
 static int check_params(lyap_ctx *ctx, const LyapParams *prm, const int32_t *seq,
-                        EvalDesc *e, uint32_t renorm)
+                        EvalDesc *e)
 {
     if (!prm || !seq) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "null parameters or sequence");
-    if (!make_eval_desc(e, *prm, seq, renorm))
+    if (!make_eval_desc(e, *prm, seq))
         return fail(ctx, LYAP_ERR_BAD_SEQUENCE,
                     "sequence must hold 1..%d letter indices 0..3 before the -1",
                     LYAP_MAX_SEQ);
@@ -224,7 +224,7 @@ int lyap_calc_volume(lyap_ctx *ctx, float *d_exps, const LyapParams *prm,
     if ((uint64_t)nx * ny * nz == 0) return LYAP_OK;
     if (!d_exps) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "null output");
     EvalDesc e;
-    int rc = check_params(ctx, prm, seq, &e, mode.renorm);
+    int rc = check_params(ctx, prm, seq, &e);
     if (rc) return rc;
     return launch_volume(ctx, d_exps, e, lo, hi, nx, ny, nz, nullptr, 0, mode);
 }
@@ -243,7 +243,7 @@ int lyap_calc_volume_noalloc(lyap_ctx *ctx, float *d_exps, const LyapParams *prm
     if ((uint64_t)nx * ny * nz == 0) return LYAP_OK;
     if (!d_exps) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "null output");
     EvalDesc e;
-    int rc = check_params(ctx, prm, seq, &e, mode.renorm);
+    int rc = check_params(ctx, prm, seq, &e);
     if (rc) return rc;
     return launch_volume_noalloc(ctx, d_exps, e, lo, hi, nx, ny, nz, mode);
 }
@@ -260,7 +260,7 @@ int lyap_calc_points(lyap_ctx *ctx, float *d_out, const float *d_xyz, size_t n,
     if (n == 0) return LYAP_OK;
     if (!d_out || !d_xyz) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "null buffer");
     EvalDesc e;
-    int rc = check_params(ctx, prm, seq, &e, mode.renorm);
+    int rc = check_params(ctx, prm, seq, &e);
     if (rc) return rc;
     const float zero[3] = {0, 0, 0};
     return launch_volume(ctx, d_out, e, zero, zero, 0, 0, 0, d_xyz, n, mode);
@@ -270,12 +270,13 @@ int lyap_calc_points_halves(lyap_ctx *ctx, float *d_lambda, float *d_half1, floa
                             const float *d_xyz, size_t n, const LyapParams *prm,
                             const int32_t *seq, unsigned renorm)
 {
+    (void)renorm;   /* results do not depend on it */
     if (!ctx) return LYAP_ERR_INVALID_ARGUMENT;
     if (n == 0) return LYAP_OK;
     if (!d_lambda || !d_half1 || !d_half2 || !d_xyz)
         return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "null buffer");
     EvalDesc e;
-    int rc = check_params(ctx, prm, seq, &e, renorm);
+    int rc = check_params(ctx, prm, seq, &e);
     if (rc) return rc;
     return launch_points_halves(ctx, d_lambda, d_half1, d_half2, e, d_xyz, n);
 }
@@ -284,7 +285,8 @@ int lyap_last_reevaluated(lyap_ctx *ctx, uint64_t *count)
 {
     if (!ctx || !count) return LYAP_ERR_INVALID_ARGUMENT;
     uint32_t c = 0;
-    LYAP_HIP(ctx, hipMemcpyAsync(&c, ctx->counters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
+    if (ctx->has_reevaluated)
+        LYAP_HIP(ctx, hipMemcpyAsync(&c, ctx->counters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
     LYAP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     *count = c;
     return LYAP_OK;

@@ -26,6 +26,7 @@ struct lyap_ctx {
     uint32_t *counters = nullptr;
     uint32_t *reeval_list = nullptr;   /* voxel indices for the FP64 pass */
     size_t reeval_cap = 0;             /* entries */
+    bool has_reevaluated = false;      /* the last volume call had a rule: counters[0] holds its count */
 
     /* the render path's launch resources (render.hip) */
     void *render_res = nullptr;

@@ -19,7 +19,7 @@
  *              r_n u_{n+1}. |u| <= 1 while 0 <= r <= 4, so the running product
  *              M of |u| only shrinks between renormalisations: it is carried
  *              as an FP32 mantissa plus an int32 exponent, renormalised every
- *              block of whole periods (up to 32 steps for the volumes, one
+ *              block of whole periods (up to 40 steps for the volumes, one
  *              16- or 32-slot window for the render), and a block that ends
  *              below the smallest normal float (where gradual underflow could
  *              have cost bits) is recomputed with a renormalisation per step.
@@ -61,18 +61,27 @@ constexpr double kLn2 = 0.693147180559945309417232121458;
  * recomputed with a renormalisation per step. */
 constexpr float kUnderflowGuard = 0x1p-126f;
 
-/* The per-period volume kernels redo a block that ended at infinity (or
- * NaN) as well: the orbit of a point with r > 4 (a volume reaching past 4)
- * can escape [0, 1], and then |u| > 1 grows fast and may overflow between
- * renormalisations where its factors are finite. Redone per step the product
- * stays finite while its factors are, so their adaptive block lengths never
- * change a bit, and lambda is finite exactly when every factor is (as with
- * the reference's sum of logs). The window forms of the persistent launch
- * keep the one compare: their samples lie in the [lMin, lMax] box (at most
- * an ulp past it), and this check costs the render kernels registers. */
-__device__ __forceinline__ bool redo_block(float M)
+/* The per-period kernels keep the running product scaled by 2^120 within a
+ * block of steps: |u| <= 1 only shrinks it, so a block has 2^246 of range
+ * before gradual underflow could cost bits, and scaling by a power of two is
+ * exact. (Started at [0.5, 1), 30-step blocks in stable regions fell below
+ * 2^-126 about half the time.) */
+constexpr float kProductScale = 0x1p120f;
+constexpr int kProductScaleExp = 120;
+
+/* Whether a block's product has to be redone: it ended below the smallest
+ * normal float, where bits may be lost, or at infinity or NaN (the orbit of a
+ * point with r > 4, in a volume reaching past 4, can escape [0, 1], and then
+ * |u| > 1 grows fast and may overflow between renormalisations where its
+ * factors are finite). Redone per step the product stays finite while its
+ * factors are, so block lengths never change a bit, and lambda is finite
+ * exactly when every factor is (as with the reference's sum of logs). One
+ * compare: the class is not "positive normal". The window forms of the
+ * persistent launch keep a compare with the guard: their samples lie in the
+ * [lMin, lMax] box (at most an ulp past it). */
+__device__ __forceinline__ bool bad_block(float M)
 {
-    return !(M >= kUnderflowGuard && M <= 0x1.fffffep127f);
+    return !__builtin_amdgcn_classf(M, 0x100);
 }
 
 /* Wave-uniform description of one lambda evaluation: iteration counts,
@@ -91,10 +100,6 @@ struct EvalDesc {
     /* first part of the window for the convergence check: the head plus
      * half_periods full periods (half_steps steps) */
     uint32_t half_periods, half_steps;
-    /* product form: full periods per renormalisation block, and after a
-     * block that had to be redone */
-    uint32_t block_periods;
-    uint32_t block_short;
     /* occurrences of letters A..D in the whole window and in its first part */
     float count[4];
     float count_half[4];
@@ -116,18 +121,8 @@ struct EvalDesc {
 
 inline void rebuild_blocks(EvalDesc *e, uint32_t W);
 
-/* Default product blocks of the per-period volume kernels: whole periods
- * making up to kBlockLong steps, and after the first block that had to be
- * redone (see redo_block) the whole periods nearest kBlockShort. The whole wave waits for any
- * lane's redo: where lambda is strongly negative (the stable regions of the
- * [2,4]^3 volumes) 30-step blocks redo about half the time and 10-step ones
- * rarely, while in chaotic regions long blocks redo as rarely and
- * renormalise less often. */
-constexpr uint32_t kBlockLong = 32, kBlockShort = 12;
-
 /* Host: derive the loop bounds. Returns false for an unusable sequence. */
-inline bool make_eval_desc(EvalDesc *e, const LyapParams &prm,
-                           const int32_t *seq, uint32_t renorm)
+inline bool make_eval_desc(EvalDesc *e, const LyapParams &prm, const int32_t *seq)
 {
     const int L = sequence_period(seq);
     if (L == 0) return false;
@@ -152,11 +147,6 @@ inline bool make_eval_desc(EvalDesc *e, const LyapParams &prm,
     e->tail = left % L;
     e->half_periods = e->acc_periods / 2;
     e->half_steps = (e->head_end - e->head_begin) + e->half_periods * (uint32_t)L;
-    uint32_t bp = (renorm ? renorm : kBlockLong) / (uint32_t)L;
-    e->block_periods = bp ? bp : 1;
-    /* an explicit length stays; the default shortens after a redo */
-    bp = renorm ? e->block_periods : (kBlockShort + (uint32_t)L / 2u) / (uint32_t)L;
-    e->block_short = bp ? bp : 1;
     /* letter counts */
     for (int k = 0; k < 4; ++k) { e->count[k] = 0.f; e->count_half[k] = 0.f; }
     for (uint32_t j = e->head_begin; j < e->head_end; ++j) {
@@ -201,23 +191,55 @@ inline void rebuild_blocks(EvalDesc *e, uint32_t W)
     e->acc_rem = left % e->B;
 }
 
-/* Lane's value of sequence letter `s` (0..3 = x, y, z, d); s is uniform. */
-__device__ __forceinline__ float pick(int s, float x, float y, float z, float d)
+/* Lane's value of the letter at position j, from the letter masks (uniform;
+ * one scalar load for all positions): a bit-field insert per letter, its mask
+ * the position's bit spread over a scalar register. */
+__device__ __forceinline__ void load_masks(uint32_t (&m)[4], const EvalDesc &e)
 {
-    return s == 0 ? x : (s == 1 ? y : (s == 2 ? z : d));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m[k] = e.wmask[k];
 }
-__device__ __forceinline__ double pickd(int s, double x, double y, double z,
-                                        double d)
+__device__ __forceinline__ uint32_t spread_bit(uint32_t m, int j)
 {
-    return s == 0 ? x : (s == 1 ? y : (s == 2 ? z : d));
+    return (uint32_t)((int32_t)(m << (31 - j)) >> 31);
+}
+__device__ __forceinline__ float pick_mask(const uint32_t (&m)[4], int j, float x, float y, float z, float d)
+{
+    const uint32_t ma = spread_bit(m[0], j), mb = spread_bit(m[1], j), mc = spread_bit(m[2], j);
+    uint32_t v = (__float_as_uint(z) & mc) | (__float_as_uint(d) & ~mc);
+    v = (__float_as_uint(y) & mb) | (v & ~mb);
+    v = (__float_as_uint(x) & ma) | (v & ~ma);
+    return __uint_as_float(v);
 }
 
-/* Lane's value of the letter at window position j, from the letter masks
- * (uniform); one scalar load for the whole window. */
-template <typename T>
-__device__ __forceinline__ T pick_mask(const uint32_t (&m)[4], int j, T x, T y, T z, T d)
+/* ---- blocks of periods and settled orbits -------------------------------
+ *
+ * The per-period kernels run blocks of block_periods<L>() whole periods, a
+ * power of two of them. The map is a function of the iterate alone at a given
+ * sequence position, so an iterate that comes back bit for bit to where it was
+ * a block earlier repeats that block for ever: in the stable regions the
+ * rounded orbit reaches its attractor exactly after about 24 ln 2 / |lambda|
+ * steps (53 in double), and an attractor of 1, 2, 4, ... periods divides the
+ * block. Once that is so in every lane of a wave the wave skips the rest of
+ * the settle, and in the accumulation applies the block's factors (product
+ * form), logs (plain) or derivatives (double), kept from one run of the
+ * block, without iterating the map: the same operations on the accumulator in
+ * the same order, so the same bits, in one instruction a step instead of three
+ * (product) or five (plain, double). Of the 256^3 volume over [2.5, 4]^3 47 % of the voxels and 35 % of
+ * the 4x4x4 bricks have settled by step 256, 61 % and 44 % by the end. */
+template <int L>
+constexpr int block_periods()
 {
-    return ((m[0] >> j) & 1u) ? x : (((m[1] >> j) & 1u) ? y : (((m[2] >> j) & 1u) ? z : d));
+    int h = 1;
+    while (2 * h * L <= 40) h *= 2;
+    return h;
+}
+
+/* Whether every lane's iterate came back to where the block started. */
+template <typename T>
+__device__ __forceinline__ bool settled(T now, T before)
+{
+    return __ballot(now != before) == 0;
 }
 
 /* ---- plain FP32: one log2 per accumulated step ------------------------- */
@@ -227,9 +249,11 @@ __device__ __forceinline__ float lambda_plain(float x, float y, float z,
                                               const EvalDesc &e)
 {
     float r[L], m2r[L];
+    uint32_t m[4];
+    load_masks(m, e);
 #pragma unroll
     for (int j = 0; j < L; ++j) {
-        r[j] = pick(e.letters[j], x, y, z, e.d);
+        r[j] = pick_mask(m, j, x, y, z, e.d);
         m2r[j] = -2.0f * r[j];
     }
     float v = 0.5f;
@@ -251,13 +275,43 @@ __device__ __forceinline__ float lambda_plain(float x, float y, float z,
             s += __builtin_amdgcn_logf(__builtin_fabsf(__builtin_fmaf(m2r[j], v, r[j])));
         }
     }
-    for (uint32_t p = 0; p < e.acc_periods; ++p) {
+    /* A loop of one period: in straight lines of a block the logs of several
+     * waves meet in the quarter-rate unit (10.0 ns a step with eight waves
+     * per SIMD against 8.9). It runs in stretches, to an eighth, a quarter,
+     * half and all of the window, so that looking for a settled orbit between
+     * them costs the others nothing. */
+    constexpr uint32_t H = block_periods<L>();
+    uint32_t done = 0;
+    const auto run_to = [&](uint32_t end) {
+        for (; done < end; ++done) {
 #pragma unroll
-        for (int j = 0; j < L; ++j) {
-            v = r[j] * __builtin_fmaf(-v, v, v);
-            s += __builtin_amdgcn_logf(__builtin_fabsf(__builtin_fmaf(m2r[j], v, r[j])));
+            for (int j = 0; j < L; ++j) {
+                v = r[j] * __builtin_fmaf(-v, v, v);
+                s += __builtin_amdgcn_logf(__builtin_fabsf(__builtin_fmaf(m2r[j], v, r[j])));
+            }
+        }
+    };
+    for (uint32_t part = 8; part > 1; part >>= 1) {
+        const uint32_t end = e.acc_periods / part;
+        if (end < done + H || e.acc_periods - end < 2 * H) continue;
+        run_to(end - H);
+        const float v0 = v;
+        run_to(end);
+        if (settled(v, v0)) {
+            float lg[H * L];
+#pragma unroll
+            for (int i = 0; i < (int)H * L; ++i) {
+                v = r[i % L] * __builtin_fmaf(-v, v, v);
+                lg[i] = __builtin_amdgcn_logf(__builtin_fabsf(__builtin_fmaf(m2r[i % L], v, r[i % L])));
+            }
+            for (; done + H <= e.acc_periods; done += H) {
+#pragma unroll
+                for (int i = 0; i < (int)H * L; ++i) s += lg[i];
+            }
+            break;
         }
     }
+    run_to(e.acc_periods);
 #pragma unroll
     for (int j = 0; j < L; ++j) {
         if ((uint32_t)j < e.tail) {
@@ -319,30 +373,36 @@ __device__ __forceinline__ float umap(float u, float b)
     return __builtin_fmaf(b, __builtin_fmaf(u, u, -1.0f), 1.0f);
 }
 
-/* `n` full periods in blocks of `bp` periods, renormalising after each block
- * and recomputing a block whose product redo_block() flags; once a lane of
- * the wave has needed that, the blocks are `bshort` periods long. */
-template <int L>
-__device__ __forceinline__ void product_periods(float &u, ProductState &st,
-                                                const float (&a)[L], const float (&b)[L],
-                                                uint32_t n, uint32_t &bp, uint32_t bshort)
+/* The end of a block that started at st.M * kProductScale and ended at Mb. */
+__device__ __forceinline__ void renorm_scaled(ProductState &st, float Mb)
 {
-    for (uint32_t p = 0; p < n;) {
-        const uint32_t cnt = n - p < bp ? n - p : bp;
-        p += cnt;
+    st.E += __builtin_amdgcn_frexp_expf(Mb) - kProductScaleExp;
+    st.M = __builtin_amdgcn_frexp_mantf(Mb);
+}
+
+/* `n` full periods of the product in blocks of about 12 steps, a lane's bad
+ * block recomputed with a renormalisation per step. */
+template <int L>
+__device__ __forceinline__ void product_periods_slow(float &u, ProductState &st, const float (&a)[L],
+                                                     const float (&b)[L], uint32_t n)
+{
+    constexpr uint32_t S = L < 12 ? (12 + L / 2) / L : 1;
+    for (uint32_t left = n; left;) {
+        const uint32_t cnt = left < S ? left : S;
+        left -= cnt;
         const float u0 = u;
-        const ProductState s0 = st;
+        float M = st.M * kProductScale;
         for (uint32_t k = 0; k < cnt; ++k) {
 #pragma unroll
             for (int j = 0; j < L; ++j) {
                 u = vmap(u, a[j], b[j]);
-                st.M *= __builtin_fabsf(u);
+                M *= __builtin_fabsf(u);
             }
         }
-        const bool rd = redo_block(st.M);
-        if (rd) {
+        if (!bad_block(M)) {
+            renorm_scaled(st, M);
+        } else {
             float w = u0;
-            st = s0;
             for (uint32_t k = 0; k < cnt; ++k) {
 #pragma unroll
                 for (int j = 0; j < L; ++j) {
@@ -352,8 +412,81 @@ __device__ __forceinline__ void product_periods(float &u, ProductState &st,
                 }
             }
         }
-        if (__any(rd)) bp = bshort;
-        renorm(st);
+    }
+}
+
+/* `n` full periods of the product. Straight-line blocks with one branch each
+ * (a taken branch costs a wave about 20 clocks of instruction fetch, as much
+ * as five steps: 11.2, 7.8 and 6.0 ns a step in lines of 5, 8 and 30 steps
+ * with one wave per SIMD, 4.7, 4.4 and 3.6 ns with eight), until a lane has a
+ * bad block, the wave has settled, or less than a block is left. */
+template <int L>
+__device__ __forceinline__ void product_periods(float &u, ProductState &st, const float (&a)[L],
+                                                const float (&b)[L], uint32_t n)
+{
+    constexpr uint32_t H = block_periods<L>();
+    uint32_t left = n;
+    if (left >= H) {
+        float w[H * L];                /* the block's iterates */
+        float u0;
+        ProductState s0;
+        bool bad, cycle;
+        do {
+            u0 = u;
+            s0 = st;
+            float M = st.M * kProductScale;
+#pragma unroll
+            for (int i = 0; i < (int)H * L; ++i) {
+                w[i] = vmap(i ? w[i - 1] : u, a[i % L], b[i % L]);
+                M *= __builtin_fabsf(w[i]);
+            }
+            u = w[H * L - 1];
+            bad = __ballot(bad_block(M)) != 0;
+            cycle = settled(u, u0);
+            renorm_scaled(st, M);
+            left -= H;
+        } while (!bad & !cycle & (left >= H));
+        if (bad) {
+            /* back to the state before the block */
+            u = u0;
+            st = s0;
+            left += H;
+        } else if (cycle) {
+            while (left >= H) {
+                s0 = st;
+                float M = st.M * kProductScale;
+#pragma unroll
+                for (int i = 0; i < (int)H * L; ++i) M *= __builtin_fabsf(w[i]);
+                if (__ballot(bad_block(M)) != 0) break;
+                renorm_scaled(st, M);
+                left -= H;
+            }
+        }
+    }
+    product_periods_slow<L>(u, st, a, b, left);
+}
+
+/* `n` full settle periods, in the same straight-line blocks. */
+template <int L>
+__device__ __forceinline__ void settle_periods(float &u, const float (&a)[L], const float (&b)[L],
+                                               uint32_t n)
+{
+    constexpr uint32_t H = block_periods<L>();
+    uint32_t left = n;
+    if (left >= H) {
+        bool cycle;
+        do {
+            const float u0 = u;
+#pragma unroll
+            for (int i = 0; i < (int)H * L; ++i) u = vmap(u, a[i % L], b[i % L]);
+            cycle = settled(u, u0);
+            left -= H;
+        } while (!cycle & (left >= H));
+        if (cycle) left %= H;
+    }
+    for (; left; --left) {
+#pragma unroll
+        for (int j = 0; j < L; ++j) u = vmap(u, a[j], b[j]);
     }
 }
 
@@ -363,16 +496,15 @@ __device__ __forceinline__ ProductResult lambda_product(float x, float y,
                                                         const EvalDesc &e)
 {
     float a[L], b[L];
+    uint32_t m[4];
+    load_masks(m, e);
 #pragma unroll
     for (int j = 0; j < L; ++j) {
-        b[j] = 0.5f * pick(e.letters[j], x, y, z, e.d);
+        b[j] = 0.5f * pick_mask(m, j, x, y, z, e.d);
         a[j] = 1.0f - b[j];
     }
     float u = 0.0f;
-    for (uint32_t p = 0; p < e.settle_periods; ++p) {
-#pragma unroll
-        for (int j = 0; j < L; ++j) u = vmap(u, a[j], b[j]);
-    }
+    settle_periods<L>(u, a, b, e.settle_periods);
 #pragma unroll
     for (int j = 0; j < L; ++j)
         if ((uint32_t)j < e.settle_rem) u = vmap(u, a[j], b[j]);
@@ -396,13 +528,12 @@ __device__ __forceinline__ ProductResult lambda_product(float x, float y,
         }
     }
     ProductState st_half{1.0f, 0};
-    uint32_t bp = e.block_periods;
     if (HALVES) {
-        product_periods<L>(u, st, a, b, e.half_periods, bp, e.block_short);
+        product_periods<L>(u, st, a, b, e.half_periods);
         st_half = st;
-        product_periods<L>(u, st, a, b, e.acc_periods - e.half_periods, bp, e.block_short);
+        product_periods<L>(u, st, a, b, e.acc_periods - e.half_periods);
     } else {
-        product_periods<L>(u, st, a, b, e.acc_periods, bp, e.block_short);
+        product_periods<L>(u, st, a, b, e.acc_periods);
     }
 #pragma unroll
     for (int j = 0; j < L; ++j) {
@@ -447,15 +578,28 @@ __device__ __forceinline__ void renorm64(ProductState64 &st)
     st.M = __builtin_amdgcn_frexp_mant(st.M);
 }
 
+/* Periods of an FP64 block: a power of two of them making up to 20 steps (40
+ * registers of derivatives), at least one. */
 template <int L>
+constexpr int block_periods64()
+{
+    int h = 1;
+    while (2 * h * L <= 20) h *= 2;
+    return h;
+}
+
+/* CYCLES: look for settled orbits. The FP64 pass over a list leaves that out:
+ * its points were listed because they have not settled. */
+template <int L, bool CYCLES>
 __device__ __forceinline__ double lambda_fp64(float xf, float yf, float zf,
                                               const EvalDesc &e)
 {
-    const double x = xf, y = yf, z = zf, d = e.d;
     double r[L], m2r[L];
+    uint32_t m[4];
+    load_masks(m, e);
 #pragma unroll
     for (int j = 0; j < L; ++j) {
-        r[j] = pickd(e.letters[j], x, y, z, d);
+        r[j] = (double)pick_mask(m, j, xf, yf, zf, e.d);
         m2r[j] = -2.0 * r[j];        /* exact */
     }
     double v = 0.5;
@@ -482,15 +626,43 @@ __device__ __forceinline__ double lambda_fp64(float xf, float yf, float zf,
     /* factors are at most max|r| * max|1 - 2v|; 8 of them cannot leave the
      * double range for coordinates of float magnitude (or the orbit escapes,
      * which makes lambda NaN either way) */
-    for (uint32_t p = 0; p < e.acc_periods; ++p) {
+    constexpr uint32_t H = block_periods64<L>();
+    uint32_t done = 0;
+    const auto run_to = [&](uint32_t end) {
+        for (; done < end; ++done) {
 #pragma unroll
-        for (int j = 0; j < L; ++j) {
-            v = (r[j] * v) * (1.0 - v);
-            st.M *= __builtin_fabs(__builtin_fma(m2r[j], v, r[j]));
-            if (((j + 1) & 7) == 0) renorm64(st);
+            for (int j = 0; j < L; ++j) {
+                v = (r[j] * v) * (1.0 - v);
+                st.M *= __builtin_fabs(__builtin_fma(m2r[j], v, r[j]));
+                if (((j + 1) & 7) == 0) renorm64(st);
+            }
+            if ((L & 7) != 0) renorm64(st);
         }
-        if ((L & 7) != 0) renorm64(st);
+    };
+    for (uint32_t part = 8; CYCLES && part > 1; part >>= 1) {
+        const uint32_t end = e.acc_periods / part;
+        if (end < done + H || e.acc_periods - end < 2 * H) continue;
+        run_to(end - H);
+        const double v0 = v;
+        run_to(end);
+        if (settled(v, v0)) {
+            double f[H * L];
+#pragma unroll
+            for (int i = 0; i < (int)H * L; ++i) {
+                v = (r[i % L] * v) * (1.0 - v);
+                f[i] = __builtin_fabs(__builtin_fma(m2r[i % L], v, r[i % L]));
+            }
+            for (; done + H <= e.acc_periods; done += H) {
+#pragma unroll
+                for (int i = 0; i < (int)H * L; ++i) {
+                    st.M *= f[i];
+                    if (((i % L + 1) & 7) == 0 || (i + 1) % L == 0) renorm64(st);
+                }
+            }
+            break;
+        }
     }
+    run_to(e.acc_periods);
 #pragma unroll
     for (int j = 0; j < L; ++j) {
         if ((uint32_t)j < e.tail) {
@@ -535,11 +707,10 @@ __device__ __forceinline__ void load_half_r(Coefs<W, VOL> &c, float x, float y,
 {
     const float hx = 0.5f * x, hy = 0.5f * y, hz = 0.5f * z, hd = 0.5f * e.d;
     uint32_t m[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) m[k] = e.wmask[k];
+    load_masks(m, e);
 #pragma unroll
     for (int j = 0; j < W; ++j) {
-        c.b[j] = pick_mask<float>(m, j, hx, hy, hz, hd);
+        c.b[j] = pick_mask(m, j, hx, hy, hz, hd);
         if constexpr (VOL) c.a[j] = 1.0f - c.b[j];
     }
 }
@@ -917,10 +1088,9 @@ __device__ __forceinline__ float lambda_plain_w(float x, float y, float z,
 {
     float r[W];
     uint32_t m[4];
+    load_masks(m, e);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) m[k] = e.wmask[k];
-#pragma unroll
-    for (int j = 0; j < W; ++j) r[j] = pick_mask<float>(m, j, x, y, z, e.d);
+    for (int j = 0; j < W; ++j) r[j] = pick_mask(m, j, x, y, z, e.d);
     float v = 0.5f, s = 0.0f;
     {
         PlainFull<W, false> f{v, s, r, e.set_blocks};
@@ -1050,13 +1220,11 @@ __device__ __forceinline__ double lambda_fp64_w(float xf, float yf, float zf,
                                                 const EvalDesc &e)
 {
     double r[W], m2r[W];
-    const double x = xf, y = yf, z = zf, d = e.d;
     uint32_t m[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) m[k] = e.wmask[k];
+    load_masks(m, e);
 #pragma unroll
     for (int j = 0; j < W; ++j) {
-        r[j] = pick_mask<double>(m, j, x, y, z, d);
+        r[j] = (double)pick_mask(m, j, xf, yf, zf, e.d);
         m2r[j] = -2.0 * r[j];
     }
     double v = 0.5;

@@ -2532,7 +2532,7 @@ static int view_from_api(lyap_ctx *ctx, ViewDesc &v, const LyapView &in, const L
     if (in.num_lights > LYAP_MAX_LIGHTS) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "more than %d lights", LYAP_MAX_LIGHTS);
     if (in.num_lights > 0 && !in.lights) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "null lights");
     EvalDesc e;
-    if (!make_eval_desc(&e, in.prm, in.seq, 16))
+    if (!make_eval_desc(&e, in.prm, in.seq))
         return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "sequence must hold 1..%d letter indices 0..3 before the -1", LYAP_MAX_SEQ);
     fill_view(v, e, in.cam, in.prm, in.width, in.height, in.rgba, in.points, in.depth,
               in.lambda, in.evals, in.lights, in.num_lights, mode);
@@ -2580,7 +2580,7 @@ static int append_blocks(lyap_ctx *ctx, const LyapVolumeBlock *in, unsigned n,
             return fail(ctx, LYAP_ERR_UNSUPPORTED, "volume block %u: more than 2^32-1 voxels", i);
         if (!b.out) return fail(ctx, LYAP_ERR_INVALID_ARGUMENT, "volume block %u: null output", i);
         EvalDesc e;
-        if (!make_eval_desc(&e, b.prm, b.seq, vmode.renorm))
+        if (!make_eval_desc(&e, b.prm, b.seq))
             return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "volume block %u: sequence must hold 1..%d letter "
                         "indices 0..3 before the -1", i, LYAP_MAX_SEQ);
         ViewDesc v;
@@ -2754,7 +2754,7 @@ extern "C" int lyap_calc_render(lyap_ctx *ctx, LyapRGBA *d_rgba, LyapPoint *d_po
     int rc = check_mode(ctx, mode_in, mode);
     if (rc) return rc;
     EvalDesc e;
-    if (!make_eval_desc(&e, *prm, seq, 16))
+    if (!make_eval_desc(&e, *prm, seq))
         return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "sequence must hold 1..%d letter indices 0..3 before the -1", LYAP_MAX_SEQ);
     return launch_render(ctx, d_rgba, d_points, *cam, *prm, e, d_lights, num_lights,
                          w, h, d_depth, d_lambda, d_evals, mode);
@@ -2859,7 +2859,7 @@ static int run_blocks_apart(lyap_ctx *ctx, const LyapVolumeBlock *blocks, unsign
     for (unsigned i = 0; i < n; ++i) {
         const LyapVolumeBlock &b = blocks[i];
         EvalDesc e;
-        if (!make_eval_desc(&e, b.prm, b.seq, vmode.renorm))
+        if (!make_eval_desc(&e, b.prm, b.seq))
             return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "volume block %u: bad sequence", i);
         const uint32_t z1 = b.z_end ? b.z_end : b.n[2];
         int rc = launch_volume_slab(ctx, b.out, e, b.lo, b.hi, b.n[0], b.n[1], b.n[2], b.z_begin, z1,

@@ -151,13 +151,15 @@ private:
             for (size_t b = 0; b < l.blocks.size(); ++b) {
                 const LyapVolumeBlock &k = l.blocks[b];
                 EvalDesc e;
-                if (!make_eval_desc(&e, k.prm, k.seq, cfg_.vol_mode.renorm))
+                if (!make_eval_desc(&e, k.prm, k.seq))
                     return fail(sl.ctx, LYAP_ERR_BAD_SEQUENCE, "bad sequence");
                 int rc = launch_volume_slab(sl.ctx, k.out, e, k.lo, k.hi, k.n[0], k.n[1], k.n[2], k.z_begin,
                                             k.z_end, nullptr, 0, cfg_.vol_mode);
                 if (rc) return rc;
-                LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval + b * kItemCountStride, sl.ctx->counters, 4,
-                                                hipMemcpyDeviceToHost, sl.ctx->stream));
+                sl.host_reeval[b * kItemCountStride] = 0;
+                if (sl.ctx->has_reevaluated)
+                    LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval + b * kItemCountStride, sl.ctx->counters, 4,
+                                                    hipMemcpyDeviceToHost, sl.ctx->stream));
             }
             *sl.host_evals = l.voxels;
         } else {
