@@ -53,6 +53,8 @@ void ctx_free(lyap_ctx *ctx, void *ptr)
 
 int ensure_reeval_list(lyap_ctx *ctx, size_t entries)
 {
+    /* parts of equal size */
+    entries = (entries + kReevalParts - 1) / kReevalParts * kReevalParts;
     if (entries <= ctx->reeval_cap) return LYAP_OK;
     LYAP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     ctx_free(ctx, ctx->reeval_list);
@@ -133,7 +135,7 @@ int lyap_create(lyap_ctx **out, int device, size_t hbm_budget_bytes)
     hipDeviceProp_t props;
     if (hipGetDeviceProperties(&props, device) == hipSuccess) ctx->num_cus = props.multiProcessorCount;
     void *p = nullptr;
-    if (ctx_alloc(ctx, &p, 256) != LYAP_OK) {
+    if (ctx_alloc(ctx, &p, (kReevalWords + 1) * sizeof(uint32_t)) != LYAP_OK) {
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return LYAP_ERR_DEVICE;
@@ -142,7 +144,7 @@ int lyap_create(lyap_ctx **out, int device, size_t hbm_budget_bytes)
     /* the allocation-free entry's scratch address on this device; a failure
      * is reported by that entry alone */
     (void)noalloc_scratch_setup(device);
-    if (launch_zero_u32(ctx, ctx->counters, 64) != LYAP_OK ||
+    if (launch_zero_u32(ctx, ctx->counters, kReevalWords + 1) != LYAP_OK ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
         lyap_destroy(ctx);
         return LYAP_ERR_DEVICE;
@@ -286,7 +288,7 @@ int lyap_last_reevaluated(lyap_ctx *ctx, uint64_t *count)
     if (!ctx || !count) return LYAP_ERR_INVALID_ARGUMENT;
     uint32_t c = 0;
     if (ctx->has_reevaluated)
-        LYAP_HIP(ctx, hipMemcpyAsync(&c, ctx->counters, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
+        LYAP_HIP(ctx, hipMemcpyAsync(&c, ctx->counters + kReevalWords, sizeof(c), hipMemcpyDeviceToHost, ctx->stream));
     LYAP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     *count = c;
     return LYAP_OK;

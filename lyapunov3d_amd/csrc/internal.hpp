@@ -22,11 +22,12 @@ struct lyap_ctx {
     std::string last_error;
     std::unordered_map<void *, size_t> allocations;
 
-    /* scratch: [0] FP64 re-evaluation count */
+    /* scratch: counters of the FP64 re-evaluation list's parts, then (word
+     * kReevalWords) the entries of the last list */
     uint32_t *counters = nullptr;
     uint32_t *reeval_list = nullptr;   /* voxel indices for the FP64 pass */
     size_t reeval_cap = 0;             /* entries */
-    bool has_reevaluated = false;      /* the last volume call had a rule: counters[0] holds its count */
+    bool has_reevaluated = false;      /* the last volume call had a rule, and so a list */
 
     /* the render path's launch resources (render.hip) */
     void *render_res = nullptr;
@@ -50,6 +51,19 @@ int fail(lyap_ctx *ctx, int code, const char *fmt, ...);
 int ctx_alloc(lyap_ctx *ctx, void **ptr, size_t bytes);
 void ctx_free(lyap_ctx *ctx, void *ptr);
 
+/* The FP64 re-evaluation list is kReevalParts parts with a counter each on a
+ * 128-byte line. A device-scope atomic takes 10 to 20 ns on its address, one
+ * after the other: with one counter the 29,600 waves of a 154 x 184 x 67
+ * volume at 464 iterations queued for 343 us (72 us with these). */
+constexpr uint32_t kReevalParts = 64;
+constexpr uint32_t kReevalStride = 32;            /* words */
+constexpr uint32_t kReevalWords = kReevalParts * kReevalStride;
+/* Whether the mode re-evaluates voxels in FP64. */
+inline bool has_rule(const LyapVolumeMode &m)
+{
+    return m.precision == LYAP_PREC_PRODUCT && (m.fp64_margin > 0.0f || m.converge_tau > 0.0f);
+}
+
 int ensure_reeval_list(lyap_ctx *ctx, size_t entries);
 
 /* Records the next timing event on the context's stream (no-op when timing
@@ -66,10 +80,13 @@ int launch_volume(lyap_ctx *ctx, float *out, const EvalDesc &e,
 
 void free_render_resources(lyap_ctx *ctx);
 
+/* z slices [z_begin, z_end) of a grid. With a rule the voxels re-evaluated are
+ * counted in *total (device memory; null: the context's word). */
 int launch_volume_slab(lyap_ctx *ctx, float *out, const EvalDesc &e,
                        const float lo[3], const float hi[3], unsigned nx,
                        unsigned ny, unsigned nz, unsigned z_begin, unsigned z_end,
-                       const float *xyz, size_t npoints, const LyapVolumeMode &mode);
+                       const float *xyz, size_t npoints, const LyapVolumeMode &mode,
+                       uint32_t *total = nullptr);
 
 /* The allocation-free volume path: entries of its scratch list (16 MiB). */
 constexpr uint32_t kNoAllocListCap = 1u << 22;

@@ -589,7 +589,8 @@ constexpr int block_periods64()
 }
 
 /* CYCLES: look for settled orbits. The FP64 pass over a list leaves that out:
- * its points were listed because they have not settled. */
+ * its points were listed because they have not settled (and the derivatives
+ * kept cost it a wave per SIMD: 2.34 ms against 2.30 for 6.1 M points). */
 template <int L, bool CYCLES>
 __device__ __forceinline__ double lambda_fp64(float xf, float yf, float zf,
                                               const EvalDesc &e)

@@ -158,7 +158,7 @@ private:
                 if (rc) return rc;
                 sl.host_reeval[b * kItemCountStride] = 0;
                 if (sl.ctx->has_reevaluated)
-                    LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval + b * kItemCountStride, sl.ctx->counters, 4,
+                    LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval + b * kItemCountStride, sl.ctx->counters + kReevalWords, 4,
                                                     hipMemcpyDeviceToHost, sl.ctx->stream));
             }
             *sl.host_evals = l.voxels;

@@ -21,6 +21,7 @@
 #include <mutex>
 
 #include "internal.hpp"
+#include "lists.hpp"
 
 namespace lyap {
 namespace {
@@ -35,10 +36,11 @@ struct VolumeArgs {
      * 64 voxels in memory order */
     uint32_t sx, sy, gx, gy, gz;
     float lo[3], span[3];
-    uint32_t *list;            /* FP64 re-evaluation list */
-    uint32_t *count;
+    uint32_t *list;            /* FP64 re-evaluation list: kReevalParts parts of `part` entries */
+    uint32_t *count;           /* their counters, kReevalStride words apart */
+    uint32_t *total;           /* entries of the list */
     float margin, tau, band;
-    uint32_t list_cap;
+    uint32_t part;
     EvalDesc e;
 };
 
@@ -78,9 +80,11 @@ __device__ __forceinline__ bool lane_voxel(const VolumeArgs &a, uint64_t &idx, f
         voxel_coords(a, idx, x, y, z);
         return true;
     }
-    /* runs of 16 bricks on one XCD (block index modulo 8) */
+    /* runs of 4 bricks on one XCD (block index modulo 8), another XCD each
+     * time, so that no XCD keeps one part of the box: with fixed runs of 16,
+     * a quarter row, the XCDs with the chaotic quarter ran a quarter longer */
     const uint32_t b = blockIdx.x;
-    const uint32_t g = (b & ~127u) + (b & 7u) * 16u + ((b >> 3) & 15u);
+    const uint32_t g = (b & ~31u) + ((b + (b >> 5)) & 7u) * 4u + ((b >> 3) & 3u);
     const uint32_t row = g / a.gx, bx = g - row * a.gx;
     const uint32_t bz = row / a.gy, by = row - bz * a.gy;
     const uint32_t sz = 6u - a.sx - a.sy;
@@ -94,19 +98,27 @@ __device__ __forceinline__ bool lane_voxel(const VolumeArgs &a, uint64_t &idx, f
 }
 
 /* Appends idx to the list for every lane with `want` set: one atomic per
- * wave, ranks from the ballot. */
+ * wave on its part's counter, ranks from the ballot. Voxels that do not fit
+ * go on to the next part: the parts hold the launch's voxels together, and a
+ * full part has every one of its entries written, so each voxel finds one. */
 __device__ __forceinline__ void append_list(const VolumeArgs &a, bool want,
                                             uint32_t idx)
 {
-    const uint64_t mask = __ballot(want);
-    if (mask == 0) return;
-    const int leader = __ffsll((unsigned long long)mask) - 1;
-    uint32_t base = 0;
-    if ((int)__lane_id() == leader) base = atomicAdd(a.count, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    if (want) {
-        const uint32_t slot = base + (uint32_t)__popcll(mask & __lanemask_lt());
-        if (slot < a.list_cap) a.list[slot] = idx;
+    for (uint32_t tries = 0; tries < kReevalParts; ++tries) {
+        const uint64_t mask = __ballot(want);
+        if (mask == 0) return;
+        const uint32_t p = (blockIdx.x + tries) % kReevalParts;
+        const int leader = __ffsll((unsigned long long)mask) - 1;
+        uint32_t base = 0;
+        if ((int)__lane_id() == leader) base = atomicAdd(a.count + p * kReevalStride, (uint32_t)__popcll(mask));
+        base = __shfl(base, leader);
+        if (want) {
+            const uint32_t slot = base + (uint32_t)__popcll(mask & __lanemask_lt());
+            if (slot < a.part) {
+                a.list[(uint64_t)p * a.part + slot] = idx;
+                want = false;
+            }
+        }
     }
 }
 
@@ -146,16 +158,30 @@ __global__ __launch_bounds__(64) void volume_fp64(VolumeArgs a)
     a.out[idx] = (float)lambda_fp64<L, true>(x, y, z, a.e);
 }
 
-/* FP64 pass over the list. */
+/* FP64 pass over the list, a wave per 64 entries of a part. */
+static_assert(kReevalParts == 64, "a lane per part");
 template <int L>
 __global__ __launch_bounds__(256) void list_fp64(VolumeArgs a)
 {
-    const uint32_t total = min(*a.count, a.list_cap);
-    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < total; i += (uint64_t)gridDim.x * 256u) {
-        const uint32_t idx = a.list[i];
-        float x, y, z;
-        voxel_coords(a, idx, x, y, z);
-        a.out[idx] = (float)lambda_fp64<L, false>(x, y, z, a.e);
+    const uint32_t lane = __lane_id();
+    const uint32_t n = min(a.count[lane * kReevalStride], a.part);    /* lane j: part j */
+    const ChunkMap cm = chunk_map(n, 64u, lane);
+    const uint32_t wid = uniform(blockIdx.x * 4u + threadIdx.x / 64u);
+    if (wid == 0) {
+        uint32_t sum = n;
+        for (int off = 32; off > 0; off >>= 1) sum += (uint32_t)__shfl_xor((int)sum, off);
+        if (lane == 0) *a.total = sum;
+    }
+    for (uint32_t c = wid; c < cm.total; c += gridDim.x * 4u) {
+        uint32_t p, acc, cnt;
+        chunk_find(cm, c, 64u, p, acc, cnt);
+        const uint32_t i = (c - acc) * 64u + lane;
+        if (i < cnt) {
+            const uint32_t idx = a.list[(uint64_t)p * a.part + i];
+            float x, y, z;
+            voxel_coords(a, idx, x, y, z);
+            a.out[idx] = (float)lambda_fp64<L, false>(x, y, z, a.e);
+        }
     }
 }
 
@@ -196,7 +222,7 @@ struct VolumeLaunch {
                    bool fp64_pass)
     {
         const uint64_t bricks = (uint64_t)a.gx * a.gy * a.gz;
-        const dim3 grid((uint32_t)(bricks ? (bricks + 127) / 128 * 128 : (a.n + 63) / 64)), block(64);
+        const dim3 grid((uint32_t)(bricks ? (bricks + 31) / 32 * 32 : (a.n + 63) / 64)), block(64);
         if (precision == LYAP_PREC_PLAIN)
             hipLaunchKernelGGL(volume_plain<L>, grid, block, 0, ctx->stream, a);
         else if (precision == LYAP_PREC_FP64)
@@ -316,7 +342,7 @@ static int launch_volume_slab_in(lyap_ctx *ctx, float *out, const EvalDesc &e,
                                  const float lo[3], const float hi[3], unsigned nx,
                                  unsigned ny, unsigned nz, unsigned z_begin, unsigned z_end,
                                  const float *xyz, size_t npoints, const LyapVolumeMode &mode,
-                                 uint32_t *list, uint32_t list_cap, uint32_t *count)
+                                 uint32_t *list, uint64_t list_cap, uint32_t *count, uint32_t *total)
 {
     VolumeArgs a{};
     a.out = out;
@@ -343,15 +369,15 @@ static int launch_volume_slab_in(lyap_ctx *ctx, float *out, const EvalDesc &e,
     a.margin = mode.fp64_margin;
     a.tau = mode.converge_tau;
     a.band = mode.converge_band;
-    const bool reeval = mode.precision == LYAP_PREC_PRODUCT &&
-                        (mode.fp64_margin > 0.0f || mode.converge_tau > 0.0f);
+    const bool reeval = has_rule(mode);
     const bool halves = reeval && mode.converge_tau > 0.0f;
     if (reeval) {
-        int rc = launch_zero_u32(ctx, count, 1);
+        int rc = launch_zero_u32(ctx, count, kReevalWords);
         if (rc) return rc;
         a.count = count;
+        a.total = total;
         a.list = list;
-        a.list_cap = list_cap;
+        a.part = (uint32_t)(list_cap / kReevalParts);
     }
     switch (e.L) {
         LYAP_L_CASES(VolumeLaunch, ctx, a, mode.precision, halves, reeval)
@@ -364,29 +390,28 @@ static int launch_volume_slab_in(lyap_ctx *ctx, float *out, const EvalDesc &e,
 int launch_volume_slab(lyap_ctx *ctx, float *out, const EvalDesc &e,
                        const float lo[3], const float hi[3], unsigned nx,
                        unsigned ny, unsigned nz, unsigned z_begin, unsigned z_end,
-                       const float *xyz, size_t npoints, const LyapVolumeMode &mode)
+                       const float *xyz, size_t npoints, const LyapVolumeMode &mode, uint32_t *total)
 {
     const uint64_t n = xyz ? (uint64_t)npoints : (uint64_t)nx * ny * (z_end - z_begin);
-    const bool reeval = mode.precision == LYAP_PREC_PRODUCT &&
-                        (mode.fp64_margin > 0.0f || mode.converge_tau > 0.0f);
+    const bool reeval = has_rule(mode);
     if (reeval && n > 0 && n <= 0xFFFFFFFFull) {
         int rc = ensure_reeval_list(ctx, n);
         if (rc) return rc;
     }
     ctx->has_reevaluated = reeval;
     return launch_volume_slab_in(ctx, out, e, lo, hi, nx, ny, nz, z_begin, z_end, xyz, npoints,
-                                 mode, ctx->reeval_list, (uint32_t)ctx->reeval_cap, ctx->counters);
+                                 mode, ctx->reeval_list, ctx->reeval_cap, ctx->counters,
+                                 total ? total : ctx->counters + kReevalWords);
 }
 
 /* ---- the allocation-free volume entry ------------------------------------- */
 
-/* Scratch of lyap_calc_volume_noalloc: word 0 is the FP64 re-evaluation
- * counter (alone on its 256-byte line), the list starts at word
- * kNoAllocListOffset. One copy per device, held until the process ends. In
+/* Scratch of lyap_calc_volume_noalloc: the FP64 re-evaluation list's counters
+ * and its total first, the list from word kNoAllocListOffset on. One copy per device, held until the process ends. In
  * host code this name is only a stand-in: kernels receive the device
  * address that hipGetSymbolAddress returned for the device
  * (noalloc_scratch_setup). */
-constexpr uint32_t kNoAllocListOffset = 64;
+constexpr uint32_t kNoAllocListOffset = kReevalWords + 64;
 static __device__ __align__(256) uint32_t scratch[kNoAllocListOffset + kNoAllocListCap];
 
 namespace {
@@ -437,7 +462,8 @@ int launch_volume_noalloc(lyap_ctx *ctx, float *out, const EvalDesc &e, const fl
     for (uint32_t z = 0; z < nz; z += per) {
         const uint32_t z1 = nz - z < per ? nz : z + per;
         int rc = launch_volume_slab_in(ctx, out + plane * z, e, lo, hi, nx, ny, nz, z, z1, nullptr, 0,
-                                       mode, base + kNoAllocListOffset, kNoAllocListCap, base);
+                                       mode, base + kNoAllocListOffset, kNoAllocListCap, base,
+                                       base + kReevalWords);
         if (rc) return rc;
     }
     return LYAP_OK;
