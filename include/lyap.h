@@ -134,7 +134,7 @@ enum {
      * (kernel.cu:140-150). */
     LYAP_PREC_PLAIN = 0,
     /* FP32 iterate in u = 1 - 2x, derivative product carried as an FP32
-     * mantissa with an integer exponent, renormalised every `renorm` steps;
+     * mantissa with an integer exponent, renormalised every block of steps;
      * one log per evaluation. */
     LYAP_PREC_PRODUCT = 1,
     /* FP64 iterate with the reference's operation order (DOUBLE_REALS build). */
@@ -144,9 +144,9 @@ enum {
 /* Volume options. NULL selects {LYAP_PREC_PLAIN, no re-evaluation}. */
 typedef struct LyapVolumeMode {
     int32_t precision;      /* LYAP_PREC_* */
-    uint32_t renorm;        /* PRODUCT: steps between renormalisations; 0 = whole
-                               periods up to 32 steps, about 12 once a wave has
-                               had to redo a block (results do not depend on it) */
+    uint32_t renorm;        /* PRODUCT: not used (the product is renormalised after
+                               blocks of whole periods of 20 to 40 steps; results
+                               do not depend on where) */
     float fp64_margin;      /* re-evaluate in FP64 where |lambda| < margin; 0 = off */
     float converge_tau;     /* also re-evaluate where the two halves of the window */
     float converge_band;    /*   differ by > tau and the smaller half-lambda < band */
@@ -221,14 +221,15 @@ typedef struct LyapRenderMode {
     uint32_t reserved;
 } LyapRenderMode;
 
-/* How rays are spread over lanes. BATCHED: the persistent work queue with
- * lane groups per ray, refill of finished lanes and continuation launches;
- * with bisection, rays whose march found its opaque sample are refined in a
- * launch of their own, two lanes per ray. A small launch of up to 16 views
- * refined by bisection (fewer rays than about two per resident lane) marches in passes
- * instead: a set-up launch lists the rays that meet the box, then launches
- * of one round each give every listed ray K lanes (4, 8, 16, 32, then 64
- * samples at once), the last running its rays to the end of their march.
+/* How rays are spread over lanes. BATCHED: up to 64 views refined by
+ * bisection march in passes: a set-up launch takes every ray's first sample
+ * and lists those still marching, then each launch gives every listed ray K
+ * lanes (its next K samples at once, more where few rays are left) for some
+ * rounds, the last running its rays to the end of their march, and a last
+ * launch refines the rays that found their opaque sample, with one or two
+ * lanes per ray. A shape asked for through LyapTuning or lanes_per_ray, other
+ * refinements and more views run a persistent work queue with lane groups per
+ * ray, refill of finished lanes and continuation launches.
  * Views refined by the walk with step jitter run one lane per ray from the
  * first sample to the last (the next step needs the last sample's lambda).
  * LEVELS: BATCHED without the passes (the persistent launches only).
@@ -323,8 +324,8 @@ typedef struct LyapTuning {
     uint32_t level_budget[3];  /* march samples a ray may take in launch levels 0, 1
                                   and 2 before it is handed to the next level (0: 24
                                   at four or more lanes per ray, else 64 / 64 / 128) */
-    uint32_t voxel_tile;       /* voxels per work-queue claim of a volume block,
-                                  rounded up to a multiple of 64 (0: 256) */
+    uint32_t voxel_tile;       /* not used: volume blocks run in the volume kernels,
+                                  which have no claims */
 } LyapTuning;
 
 /* Renders n_views views in one persistent launch fed by a device work queue
@@ -344,16 +345,12 @@ typedef struct LyapVolumeBlock {
     float *out;
 } LyapVolumeBlock;
 
-/* Views and volume blocks of different sizes in one persistent launch
- * sequence (kernel_calc_render and kernel_calc_volume, kernel.hpp:17,19,
- * in one): the first launch's device work queue deals the views' ray tiles
- * and then the blocks' voxel tiles (one lane per voxel), so waves whose
- * rays have ended take voxels; voxels the volume mode's rule lists are
- * re-evaluated in FP64 by the next launch. Each view gets the bytes
- * lyap_calc_render gives it and each block the bytes of lyap_calc_volume
- * over the same grid (the same arithmetic). Blocks are evaluated in the
- * views' precision: when vol_mode's precision differs they run in the
- * volume kernels after the views' launches (same results, not fused). */
+/* Views and volume blocks of different sizes in one launch sequence
+ * (kernel_calc_render and kernel_calc_volume, kernel.hpp:17,19, in one): the
+ * views as lyap_render_batch, then the blocks through the volume kernels, on
+ * the context's stream. Each view gets the bytes lyap_calc_render gives it
+ * and each block the bytes of lyap_calc_volume over the same grid, whatever
+ * the precisions of the two modes. */
 int lyap_run_batch(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
                    const LyapVolumeBlock *blocks, unsigned n_blocks,
                    const LyapRenderMode *mode, const LyapVolumeMode *vol_mode,
@@ -362,8 +359,7 @@ int lyap_run_batch(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
 /* Times candidate launch shapes on a representative batch and stores the
  * fastest in the context (used when a LyapTuning field is 0): lanes per
  * ray x samples per lane (one lane per ray included) x tile length, then
- * each level's march-sample budget, then (with volume blocks) the voxel
- * tile. The results do not depend on the shape. */
+ * each level's march-sample budget. The results do not depend on the shape. */
 int lyap_autotune(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
                   const LyapRenderMode *mode, LyapTuning *best);
 int lyap_autotune_batch(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
@@ -531,7 +527,7 @@ typedef struct LyapServerStats {
  * and a volume into z slabs; each launch takes the pieces of the requests
  * with the earliest deadlines, up to about `slice_ms` of device time, so a
  * request that arrives while others run joins the next launch. A launch
- * carries views and volume slabs together (one persistent launch, as
+ * carries views and volume slabs together (one launch sequence, as
  * lyap_run_batch), each slot on its own stream, so the launches' work
  * overlaps on the device. A request's outputs are admitted against
  * `hbm_budget_bytes` when its first piece is issued and stay resident until

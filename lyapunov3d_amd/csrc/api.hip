@@ -322,12 +322,15 @@ int lyap_timing_collect(lyap_ctx *ctx, double *kernel_ms, uint64_t *launches)
 int lyap_last_evals(lyap_ctx *ctx, uint64_t *count)
 {
     if (!ctx || !count) return LYAP_ERR_INVALID_ARGUMENT;
-    *count = 0;
-    if (!ctx->last_counters) return LYAP_OK;
+    *count = ctx->last_voxels;
+    if (!ctx->last_counters) {
+        LYAP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        return LYAP_OK;
+    }
     std::vector<uint64_t> words(kEvalSlots * kEvalStride);
     LYAP_HIP(ctx, hipMemcpyAsync(words.data(), ctx->last_counters, kEvalBytes, hipMemcpyDeviceToHost, ctx->stream));
     LYAP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *count = sum_evals(words.data());
+    *count += sum_evals(words.data());
     return LYAP_OK;
 }
 

@@ -32,6 +32,7 @@ struct lyap_ctx {
     /* the render path's launch resources (render.hip) */
     void *render_res = nullptr;
     uint32_t *last_counters = nullptr; /* counters of the last render launch */
+    uint64_t last_voxels = 0;          /* voxels of the last batch's blocks */
 
     LyapTuning tuned{};                /* autotuner's choice, zero = unset */
     void *debug_wave_log = nullptr;    /* per-wave render record, when set */
@@ -104,8 +105,7 @@ int launch_points_halves(lyap_ctx *ctx, float *lam, float *h1, float *h2, const 
 struct RenderSlot;
 RenderSlot *render_slot_create();
 void render_slot_destroy(lyap_ctx *ctx, RenderSlot *slot);
-/* Lambda evaluations of a launch (rays' algorithmic samples plus one per
- * voxel) are counted in kEvalSlots 64-bit words, one per 128-byte line, and
+/* Lambda evaluations of a launch (rays' algorithmic samples) are counted in kEvalSlots 64-bit words, one per 128-byte line, and
  * added up by whoever reads them: device-scope atomics on one address take
  * about 20 ns each, one after the other, and with one word the 5,000 waves of
  * a 512 x 512 frame's refinement ended in a queue (116 us; 112 us with
@@ -121,14 +121,13 @@ inline uint64_t sum_evals(const uint64_t *words)
 }
 /* The slot's counter block, which begins with those words. */
 const uint32_t *render_slot_counters(const RenderSlot *slot);
-/* FP64 re-evaluations of each item of the last launch, kItemCountStride
- * words apart (views' entries stay 0). */
-constexpr uint32_t kItemCountStride = 32;
-const uint32_t *render_slot_vox_counts(const RenderSlot *slot);
 int render_slot_launch(lyap_ctx *ctx, RenderSlot *slot, const LyapView *views,
                        const uint32_t *ray_begin, const uint32_t *ray_count, unsigned n,
-                       const LyapVolumeBlock *blocks, unsigned nb, const LyapVolumeMode &vmode,
                        const LyapRenderMode &mode, const LyapTuning &tune);
+
+/* Volume blocks through the volume kernels (render.hip). */
+int launch_blocks(lyap_ctx *ctx, const LyapVolumeBlock *blocks, unsigned n, const LyapVolumeMode &vmode,
+                  uint32_t *totals);
 
 int launch_render(lyap_ctx *ctx, LyapRGBA *rgba, LyapPoint *points,
                   const LyapCam &cam, const LyapParams &prm, const EvalDesc &e,

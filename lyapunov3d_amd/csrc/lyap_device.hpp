@@ -100,6 +100,8 @@ struct EvalDesc {
     /* first part of the window for the convergence check: the head plus
      * half_periods full periods (half_steps steps) */
     uint32_t half_periods, half_steps;
+    /* 1 / accum and 1 / steps of the window's two parts, rounded to nearest */
+    double inv_accum, inv_half1, inv_half2;
     /* occurrences of letters A..D in the whole window and in its first part */
     float count[4];
     float count_half[4];
@@ -147,6 +149,9 @@ inline bool make_eval_desc(EvalDesc *e, const LyapParams &prm, const int32_t *se
     e->tail = left % L;
     e->half_periods = e->acc_periods / 2;
     e->half_steps = (e->head_end - e->head_begin) + e->half_periods * (uint32_t)L;
+    e->inv_accum = 1.0 / (double)prm.accum;
+    e->inv_half1 = 1.0 / (double)e->half_steps;
+    e->inv_half2 = 1.0 / (double)(prm.accum - e->half_steps);
     /* letter counts */
     for (int k = 0; k < 4; ++k) { e->count[k] = 0.f; e->count_half[k] = 0.f; }
     for (uint32_t j = e->head_begin; j < e->head_end; ++j) {
@@ -336,16 +341,29 @@ __device__ __forceinline__ void renorm(ProductState &st)
     st.M = __builtin_amdgcn_frexp_mantf(st.M);
 }
 
-/* ln of the product plus the letter terms, divided by n; NaN if not finite. */
+/* a / n for a whole number n < 2^32, given y = 1 / n rounded to nearest, in 3
+ * operations instead of the division's dozen. The estimate a * y is within
+ * 1.5 ulp, its residual a - n q fits a double and so is exact, and the
+ * corrected quotient is off by less than 2^-52 ulp before it is rounded,
+ * while a / n lies at least 2^-34 ulp from any rounding boundary: the result
+ * is the correctly rounded quotient. n = 0 and a non-finite a give NaN. */
+__device__ __forceinline__ double divide_by(double a, double n, double y)
+{
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-n, q, a), y, q);
+}
+
+/* ln of the product plus the letter terms, divided by n (inv = 1 / n); NaN if
+ * not finite. */
 __device__ __forceinline__ float finish_product(const ProductState &st,
                                                 const float lg[4],
-                                                const float cnt[4], uint32_t n)
+                                                const float cnt[4], uint32_t n, double inv)
 {
     double t = (double)st.E + (double)__builtin_amdgcn_logf(st.M);
 #pragma unroll
     for (int k = 0; k < 4; ++k)
         if (cnt[k] != 0.0f) t += (double)cnt[k] * (double)lg[k];
-    const float lam = (float)(t * kLn2 / (double)n);
+    const float lam = (float)divide_by(t * kLn2, (double)n, inv);
     return __builtin_isfinite(lam) ? lam : __builtin_nanf("");
 }
 
@@ -549,7 +567,7 @@ __device__ __forceinline__ ProductResult lambda_product(float x, float y,
     lg[1] = __builtin_amdgcn_logf(__builtin_fabsf(y));
     lg[2] = __builtin_amdgcn_logf(__builtin_fabsf(z));
     lg[3] = __builtin_amdgcn_logf(__builtin_fabsf(e.d));
-    res.lam = finish_product(st, lg, e.count, e.accum);
+    res.lam = finish_product(st, lg, e.count, e.accum, e.inv_accum);
     res.half1 = res.half2 = res.lam;
     if (HALVES) {
         const uint32_t n1 = e.half_steps, n2 = e.accum - e.half_steps;
@@ -559,8 +577,8 @@ __device__ __forceinline__ ProductResult lambda_product(float x, float y,
         ProductState second;
         second.E = st.E - st_half.E;
         second.M = st.M / st_half.M;
-        res.half1 = n1 ? finish_product(st_half, lg, e.count_half, n1) : __builtin_nanf("");
-        res.half2 = n2 ? finish_product(second, lg, c2, n2) : __builtin_nanf("");
+        res.half1 = n1 ? finish_product(st_half, lg, e.count_half, n1, e.inv_half1) : __builtin_nanf("");
+        res.half2 = n2 ? finish_product(second, lg, c2, n2, e.inv_half2) : __builtin_nanf("");
     }
     return res;
 }
@@ -680,19 +698,6 @@ __device__ __forceinline__ double lambda_fp64(float xf, float yf, float zf,
 /* Period-agnostic forms: one compiled loop for every period L <= W.         */
 /* ======================================================================== */
 
-/* The coefficients of a window of W slots: b_j = r_j / 2 and, for the
- * volume form (VOL), a_j = 1 - b_j; step(j, u) is the map at slot j. */
-template <int W, bool VOL>
-struct Coefs {
-    float b[W];
-    float a[VOL ? W : 1];
-    __device__ __forceinline__ float step(int j, float u) const
-    {
-        if constexpr (VOL) return vmap(u, a[j], b[j]);
-        else return umap(u, b[j]);
-    }
-};
-
 /* Steps of a block at positions [lo, hi) (FULL: [0, B), where every block
  * has at least W/2 + 1 steps, so only the upper half is guarded). */
 template <int W, bool FULL>
@@ -702,157 +707,92 @@ __device__ __forceinline__ bool in_block(int j, uint32_t lo, uint32_t hi)
     return (uint32_t)j >= lo && (uint32_t)j < hi;
 }
 
-template <int W, bool VOL>
-__device__ __forceinline__ void load_half_r(Coefs<W, VOL> &c, float x, float y,
-                                            float z, const EvalDesc &e)
+/* The coefficients of a window of W slots, b_j = r_j / 2. */
+template <int W>
+__device__ __forceinline__ void load_half_r(float (&b)[W], float x, float y, float z, const EvalDesc &e)
 {
     const float hx = 0.5f * x, hy = 0.5f * y, hz = 0.5f * z, hd = 0.5f * e.d;
     uint32_t m[4];
     load_masks(m, e);
 #pragma unroll
-    for (int j = 0; j < W; ++j) {
-        c.b[j] = pick_mask(m, j, hx, hy, hz, hd);
-        if constexpr (VOL) c.a[j] = 1.0f - c.b[j];
-    }
+    for (int j = 0; j < W; ++j) b[j] = pick_mask(m, j, hx, hy, hz, hd);
 }
 
-template <int W, bool VOL, bool FULL>
-__device__ __forceinline__ void settle_block(float &u, const Coefs<W, VOL> &c,
-                                             uint32_t lo, uint32_t hi)
+/* Calls f.template go<N>() for n in [LO, HI], found by halving (n is
+ * wave-uniform, so each test is a scalar branch). */
+template <int LO, int HI, class F>
+__device__ __forceinline__ void with_value(uint32_t n, F &f)
 {
-#pragma unroll
-    for (int j = 0; j < W; ++j)
-        if (in_block<W, FULL>(j, lo, hi)) u = c.step(j, u);
-}
-
-template <int W, bool VOL, bool FULL>
-__device__ __forceinline__ void product_block(float &u, ProductState &st,
-                                              const Coefs<W, VOL> &c, uint32_t lo,
-                                              uint32_t hi)
-{
-    const float u0 = u;
-    const ProductState s0 = st;
-#pragma unroll
-    for (int j = 0; j < W; ++j) {
-        if (in_block<W, FULL>(j, lo, hi)) {
-            u = c.step(j, u);
-            st.M *= __builtin_fabsf(u);
-        }
+    if constexpr (LO == HI) {
+        f.template go<LO>();
+    } else {
+        constexpr int MID = (LO + HI) / 2;
+        if (n <= (uint32_t)MID) with_value<LO, MID>(n, f);
+        else with_value<MID + 1, HI>(n, f);
     }
-    if (st.M < kUnderflowGuard) {
-        /* |u| <= 1 keeps M monotone within the block, so ending above the
-         * guard means no step went below it; otherwise redo per step */
-        float w = u0;
-        st = s0;
-#pragma unroll
-        for (int j = 0; j < W; ++j) {
-            if (in_block<W, FULL>(j, lo, hi)) {
-                w = c.step(j, w);
-                st.M *= __builtin_fabsf(w);
-                renorm(st);
-            }
-        }
-    }
-    renorm(st);
 }
 
 /* Calls f.template go<B>() with B the block length Bv, one of (W/2, W]. A
- * full block then runs exactly B unguarded steps. Bv comes from the view
- * descriptor and is the same for every lane of the wave, so the choice is a
- * scalar branch. */
-template <int W, int B, class F>
+ * full block then runs exactly B unguarded steps. */
+template <int W, class F>
 __device__ __forceinline__ void with_block_len(uint32_t Bv, F &f)
 {
-    if constexpr (B > W / 2) {
-        if (Bv == (uint32_t)B) f.template go<B>();
-        else with_block_len<W, B - 1>(Bv, f);
-    }
+    with_value<W / 2 + 1, W>(Bv, f);
 }
-
-/* n full settle blocks of B steps. */
-template <int W, bool VOL>
-struct SettleFull {
-    float &u;
-    const Coefs<W, VOL> &c;
-    uint32_t n;
-    template <int B>
-    __device__ __forceinline__ void go()
-    {
-        for (uint32_t k = 0; k < n; ++k) {
-#pragma unroll
-            for (int j = 0; j < B; ++j) u = c.step(j, u);
-        }
-    }
-};
-
-/* n full product blocks of B steps, with the same underflow redo as
- * product_block. */
-template <int W, bool VOL>
-struct ProductFull {
-    float &u;
-    ProductState &st;
-    const Coefs<W, VOL> &c;
-    uint32_t n;
-    template <int B>
-    __device__ __forceinline__ void go()
-    {
-        for (uint32_t k = 0; k < n; ++k) {
-            const float u0 = u;
-            const ProductState s0 = st;
-#pragma unroll
-            for (int j = 0; j < B; ++j) {
-                u = c.step(j, u);
-                st.M *= __builtin_fabsf(u);
-            }
-            if (st.M < kUnderflowGuard) {
-                float w = u0;
-                st = s0;
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    w = c.step(j, w);
-                    st.M *= __builtin_fabsf(w);
-                    renorm(st);
-                }
-            }
-            renorm(st);
-        }
-    }
-};
 
 /* Calls f.template go<N>() for n in [1, W); nothing for n = 0. Partial
  * blocks are specialised by their start or length this way, so none of
- * their steps carries a per-step guard. n is wave-uniform. */
-template <int W, int N, class F>
+ * their steps carries a per-step guard. */
+template <int W, class F>
 __device__ __forceinline__ void with_len(uint32_t n, F &f)
 {
-    if constexpr (N >= 1) {
-        if (n == (uint32_t)N) f.template go<N>();
-        else with_len<W, N - 1>(n, f);
-    }
+    if (n != 0) with_value<1, W - 1>(n, f);
 }
 
+/* n full settle blocks of B steps. The loops of the window forms are one
+ * block long: a launch of the march starts with a cold instruction cache, and
+ * with runs of two blocks (and the redo apart from them) a 256 x 256 frame's
+ * passes took 28 % longer, fetching code they run a few times. */
+template <int W>
+struct SettleFull {
+    float &u;
+    const float (&c)[W];
+    uint32_t n;
+    template <int B>
+    __device__ __forceinline__ void go()
+    {
+        for (uint32_t k = 0; k < n; ++k) {
+#pragma unroll
+            for (int j = 0; j < B; ++j) u = umap(u, c[j]);
+        }
+    }
+};
+
 /* Window positions [LO, HI) of the product form; positions past W/2 are
- * guarded by j < hi when GUARD (they may lie past a block of B < W). */
-template <int W, bool VOL, int LO, int HI, bool GUARD>
-__device__ __forceinline__ void product_range(float &u, ProductState &st,
-                                              const Coefs<W, VOL> &c, uint32_t hi)
+ * guarded by j < hi when GUARD (they may lie past a block of B < W). A lane
+ * whose block ends below the smallest normal float redoes it with a
+ * renormalisation per step. */
+template <int W, int LO, int HI, bool GUARD>
+__device__ __forceinline__ void product_range(float &u, ProductState &st, const float (&c)[W], uint32_t hi)
 {
     const float u0 = u;
     const ProductState s0 = st;
 #pragma unroll
     for (int j = LO; j < HI; ++j) {
         if (!GUARD || j <= W / 2 || (uint32_t)j < hi) {
-            u = c.step(j, u);
+            u = umap(u, c[j]);
             st.M *= __builtin_fabsf(u);
         }
     }
     if (st.M < kUnderflowGuard) {
+        /* |u| <= 1 keeps M monotone within the block, so ending above the
+         * guard means no step went below it */
         float w = u0;
         st = s0;
 #pragma unroll
         for (int j = LO; j < HI; ++j) {
             if (!GUARD || j <= W / 2 || (uint32_t)j < hi) {
-                w = c.step(j, w);
+                w = umap(w, c[j]);
                 st.M *= __builtin_fabsf(w);
                 renorm(st);
             }
@@ -861,36 +801,79 @@ __device__ __forceinline__ void product_range(float &u, ProductState &st,
     renorm(st);
 }
 
+/* The window positions [lo, hi), any 0 <= lo <= hi <= W. */
+template <int W>
+__device__ __forceinline__ void product_block(float &u, ProductState &st, const float (&c)[W],
+                                              uint32_t lo, uint32_t hi)
+{
+    const float u0 = u;
+    const ProductState s0 = st;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        if ((uint32_t)j >= lo && (uint32_t)j < hi) {
+            u = umap(u, c[j]);
+            st.M *= __builtin_fabsf(u);
+        }
+    }
+    if (st.M < kUnderflowGuard) {
+        float w = u0;
+        st = s0;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            if ((uint32_t)j >= lo && (uint32_t)j < hi) {
+                w = umap(w, c[j]);
+                st.M *= __builtin_fabsf(w);
+                renorm(st);
+            }
+        }
+    }
+    renorm(st);
+}
+
+/* n full product blocks of B steps. */
+template <int W>
+struct ProductFull {
+    float &u;
+    ProductState &st;
+    const float (&c)[W];
+    uint32_t n;
+    template <int B>
+    __device__ __forceinline__ void go()
+    {
+        for (uint32_t k = 0; k < n; ++k) product_range<W, 0, B, false>(u, st, c, 0);
+    }
+};
+
 /* Settle steps [0, N) / product steps [0, N) / the rest of a block from N. */
-template <int W, bool VOL>
+template <int W>
 struct SettlePrefix {
     float &u;
-    const Coefs<W, VOL> &c;
+    const float (&c)[W];
     template <int N>
     __device__ __forceinline__ void go()
     {
 #pragma unroll
-        for (int j = 0; j < N; ++j) u = c.step(j, u);
+        for (int j = 0; j < N; ++j) u = umap(u, c[j]);
     }
 };
 
-template <int W, bool VOL>
+template <int W>
 struct ProductPrefix {
     float &u;
     ProductState &st;
-    const Coefs<W, VOL> &c;
+    const float (&c)[W];
     template <int N>
-    __device__ __forceinline__ void go() { product_range<W, VOL, 0, N, false>(u, st, c, 0); }
+    __device__ __forceinline__ void go() { product_range<W, 0, N, false>(u, st, c, 0); }
 };
 
-template <int W, bool VOL>
+template <int W>
 struct ProductHead {
     float &u;
     ProductState &st;
-    const Coefs<W, VOL> &c;
+    const float (&c)[W];
     uint32_t hi;
     template <int N>
-    __device__ __forceinline__ void go() { product_range<W, VOL, N, W, true>(u, st, c, hi); }
+    __device__ __forceinline__ void go() { product_range<W, N, W, true>(u, st, c, hi); }
 };
 
 /* FP32 product form, any period L <= W, with the render's map. */
@@ -898,120 +881,40 @@ template <int W>
 __device__ __forceinline__ float lambda_product_w(float x, float y, float z,
                                                   const EvalDesc &e)
 {
-    constexpr bool VOL = false;
-    Coefs<W, VOL> c;
-    load_half_r<W, VOL>(c, x, y, z, e);
+    float c[W];
+    load_half_r<W>(c, x, y, z, e);
     float u = 0.0f;
     {
-        SettleFull<W, VOL> f{u, c, e.set_blocks};
-        with_block_len<W, W>(e.B, f);
+        SettleFull<W> f{u, c, e.set_blocks};
+        with_block_len<W>(e.B, f);
     }
     {
-        SettlePrefix<W, VOL> f{u, c};
-        with_len<W, W - 1>(e.set_rem, f);
+        SettlePrefix<W> f{u, c};
+        with_len<W>(e.set_rem, f);
     }
     if (__builtin_fabsf(u) < 2e-8f) return 0.0f / (float)e.accum;   /* kernel.cu:138 */
     ProductState st{1.0f, 0};
     if (e.head_hi == e.B) {
         /* the usual head: the rest of the block the settle ended in */
-        ProductHead<W, VOL> f{u, st, c, e.B};
-        with_len<W, W - 1>(e.head_lo, f);
+        ProductHead<W> f{u, st, c, e.B};
+        with_len<W>(e.head_lo, f);
     } else {
-        product_block<W, VOL, false>(u, st, c, e.head_lo, e.head_hi);
+        product_block<W>(u, st, c, e.head_lo, e.head_hi);
     }
     {
-        ProductFull<W, VOL> f{u, st, c, e.acc_blocks};
-        with_block_len<W, W>(e.B, f);
+        ProductFull<W> f{u, st, c, e.acc_blocks};
+        with_block_len<W>(e.B, f);
     }
     {
-        ProductPrefix<W, VOL> f{u, st, c};
-        with_len<W, W - 1>(e.acc_rem, f);
+        ProductPrefix<W> f{u, st, c};
+        with_len<W>(e.acc_rem, f);
     }
     float lg[4];
     lg[0] = __builtin_amdgcn_logf(__builtin_fabsf(x));
     lg[1] = __builtin_amdgcn_logf(__builtin_fabsf(y));
     lg[2] = __builtin_amdgcn_logf(__builtin_fabsf(z));
     lg[3] = __builtin_amdgcn_logf(__builtin_fabsf(e.d));
-    return finish_product(st, lg, e.count, e.accum);
-}
-
-/* n product steps from window position p (p < B): the rest of that block,
- * whole blocks, then a prefix of one more block. Every part ends with a
- * renormalisation, which is exact, so where a run is split changes no bit
- * of the product. */
-template <int W, bool VOL>
-__device__ __forceinline__ void product_run(float &u, ProductState &st, const Coefs<W, VOL> &c,
-                                            uint32_t B, uint32_t p, uint32_t n)
-{
-    if (n == 0) return;
-    if (p != 0) {
-        const uint32_t hi = p + n < B ? p + n : B;
-        if (hi == B) {
-            ProductHead<W, VOL> f{u, st, c, B};
-            with_len<W, W - 1>(p, f);
-        } else {
-            product_block<W, VOL, false>(u, st, c, p, hi);
-        }
-        n -= hi - p;
-    }
-    {
-        ProductFull<W, VOL> f{u, st, c, n / B};
-        with_block_len<W, W>(B, f);
-    }
-    {
-        ProductPrefix<W, VOL> f{u, st, c};
-        with_len<W, W - 1>(n % B, f);
-    }
-}
-
-/* FP32 product form with the volume map, any period L <= W, with the
- * lambdas of the two parts of the window split after e.half_steps
- * accumulated steps: the same split, map and products as
- * lambda_product<L, true>, so the same bits (the products differ only in
- * where they were renormalised). */
-template <int W>
-__device__ __forceinline__ ProductResult lambda_product_halves_w(float x, float y, float z,
-                                                                 const EvalDesc &e)
-{
-    constexpr bool VOL = true;
-    Coefs<W, VOL> c;
-    load_half_r<W, VOL>(c, x, y, z, e);
-    float u = 0.0f;
-    {
-        SettleFull<W, VOL> f{u, c, e.set_blocks};
-        with_block_len<W, W>(e.B, f);
-    }
-    {
-        SettlePrefix<W, VOL> f{u, c};
-        with_len<W, W - 1>(e.set_rem, f);
-    }
-    ProductResult res;
-    if (__builtin_fabsf(u) < 2e-8f) {                 /* kernel.cu:138 */
-        res.lam = 0.0f / (float)e.accum;
-        res.half1 = res.half2 = res.lam;
-        return res;
-    }
-    ProductState st{1.0f, 0};
-    const uint32_t n1 = e.half_steps;
-    product_run<W, VOL>(u, st, c, e.B, e.set_rem, n1);
-    const ProductState st_half = st;
-    product_run<W, VOL>(u, st, c, e.B, (e.set_rem + n1) % e.B, e.accum - n1);
-    float lg[4];
-    lg[0] = __builtin_amdgcn_logf(__builtin_fabsf(x));
-    lg[1] = __builtin_amdgcn_logf(__builtin_fabsf(y));
-    lg[2] = __builtin_amdgcn_logf(__builtin_fabsf(z));
-    lg[3] = __builtin_amdgcn_logf(__builtin_fabsf(e.d));
-    res.lam = finish_product(st, lg, e.count, e.accum);
-    const uint32_t n2 = e.accum - n1;
-    float c2[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) c2[k] = e.count[k] - e.count_half[k];
-    ProductState second;
-    second.E = st.E - st_half.E;
-    second.M = st.M / st_half.M;
-    res.half1 = n1 ? finish_product(st_half, lg, e.count_half, n1) : __builtin_nanf("");
-    res.half2 = n2 ? finish_product(second, lg, c2, n2) : __builtin_nanf("");
-    return res;
+    return finish_product(st, lg, e.count, e.accum, e.inv_accum);
 }
 
 /* FP32 x-form with one log2 per accumulated step (the reference method). */
@@ -1095,26 +998,26 @@ __device__ __forceinline__ float lambda_plain_w(float x, float y, float z,
     float v = 0.5f, s = 0.0f;
     {
         PlainFull<W, false> f{v, s, r, e.set_blocks};
-        with_block_len<W, W>(e.B, f);
+        with_block_len<W>(e.B, f);
     }
     {
         PlainPrefix<W, false> f{{v, s, r, 0}};
-        with_len<W, W - 1>(e.set_rem, f);
+        with_len<W>(e.set_rem, f);
     }
     if (v == 0.5f) return 0.0f / (float)e.accum;
     if (e.head_hi == e.B) {
         PlainHead<W, true> f{{v, s, r, e.B}};
-        with_len<W, W - 1>(e.head_lo, f);
+        with_len<W>(e.head_lo, f);
     } else {
         plain_block<W, false>(v, s, r, e.head_lo, e.head_hi, true);
     }
     {
         PlainFull<W, true> f{v, s, r, e.acc_blocks};
-        with_block_len<W, W>(e.B, f);
+        with_block_len<W>(e.B, f);
     }
     {
         PlainPrefix<W, true> f{{v, s, r, 0}};
-        with_len<W, W - 1>(e.acc_rem, f);
+        with_len<W>(e.acc_rem, f);
     }
     const float lam = s * kLn2f / (float)e.accum;
     return __builtin_isfinite(lam) ? lam : __builtin_nanf("");
@@ -1233,27 +1136,27 @@ __device__ __forceinline__ double lambda_fp64_w(float xf, float yf, float zf,
     const uint32_t mid = e.B / 2u;
     {
         Fp64Full<W, false> f{v, st, r, m2r, e.set_blocks};
-        with_block_len<W, W>(e.B, f);
+        with_block_len<W>(e.B, f);
     }
     {
         Fp64Prefix<W, false> f{{v, st, r, m2r, 0, mid}};
-        with_len<W, W - 1>(e.set_rem, f);
+        with_len<W>(e.set_rem, f);
     }
     const double off = v - 0.5;
     if (!(off <= -1e-8 || off >= 1e-8)) return 0.0 / (double)e.accum;
     if (e.head_hi == e.B) {
         Fp64Head<W, true> f{{v, st, r, m2r, e.B, mid}};
-        with_len<W, W - 1>(e.head_lo, f);
+        with_len<W>(e.head_lo, f);
     } else {
         fp64_block<W, false, true>(v, st, r, m2r, e.head_lo, e.head_hi, mid);
     }
     {
         Fp64Full<W, true> f{v, st, r, m2r, e.acc_blocks};
-        with_block_len<W, W>(e.B, f);
+        with_block_len<W>(e.B, f);
     }
     {
         Fp64Prefix<W, true> f{{v, st, r, m2r, 0, mid}};
-        with_len<W, W - 1>(e.acc_rem, f);
+        with_len<W>(e.acc_rem, f);
     }
     const double lam = ((double)st.E * kLn2 + log(st.M)) / (double)e.accum;
     return __builtin_isfinite(lam) ? lam : __builtin_nan("");

@@ -4,7 +4,11 @@
  * Replaces kernel_calc_render (kernel.cu:500-516) with raymarch
  * (kernel.cu:156-486) and shade (kernel.cu:25-106) fused in.
  *
- * Schedule. The reference runs one thread per pixel, so a wave lasts as long
+ * Frames refined by bisection march in passes (march.hip) and jittered ones
+ * refined by the walk in a launch of their own (walk.hip); here are what they
+ * share, the host side, and the persistent levels for everything else.
+ *
+ * The levels. The reference runs one thread per pixel, so a wave lasts as long
  * as its slowest ray. Here every lane runs a small state machine
  * (march -> refine -> six normal samples -> shade) and each trip round the
  * kernel's main loop performs exactly one lambda evaluation per busy lane.
@@ -71,10 +75,6 @@ struct RenderArgs {
      * counters per view and sub-region, 32 words apart */
     RefineRec *refine_out;
     uint32_t *refine_counts;
-    /* volume blocks: FP64 re-evaluation list (voxel indices within a block)
-     * and its counters, per item, kHeadStride words apart */
-    uint32_t *vox_list;
-    uint32_t *vox_counts;
 };
 
 namespace {
@@ -717,70 +717,6 @@ __device__ __forceinline__ uint32_t claim_tile(uint32_t *heads, uint32_t n_waves
     return 0xFFFFFFFFu;
 }
 
-/* Coordinates of voxel i of a volume block: the volume kernels' formula
- * lo + (span * index) / n per axis (kernel.cu:527-529 for the box [0, 4)). */
-__device__ __forceinline__ void block_voxel(const ViewDesc &v, uint32_t i, float &x, float &y,
-                                            float &z)
-{
-    const uint32_t plane = v.vnx * v.vny;
-    const uint32_t lz = i / plane;
-    const uint32_t rem = i - lz * plane;
-    const uint32_t iy = rem / v.vnx;
-    const uint32_t ix = rem - iy * v.vnx;
-    x = v.vlo[0] + (v.vspan[0] * (float)ix) / (float)v.vnx;
-    y = v.vlo[1] + (v.vspan[1] * (float)iy) / (float)v.vny;
-    z = v.vlo[2] + (v.vspan[2] * (float)(v.vz0 + lz)) / (float)v.vnz;
-}
-
-/* Voxels [first, last) of volume block `item`, one lane per voxel, 64 at a
- * time, in the precision of the launch. The product form gives the same
- * bits as the volume kernels (lambda_product<L, true>) and lists the voxels
- * its rule selects (|lambda| < margin, or window halves that disagree by
- * more than tau below band) for the FP64 pass, one atomic per wave. Returns
- * the voxels this lane evaluated. */
-template <int W, int PREC>
-__device__ uint32_t voxel_tile(const ViewDesc &v, uint32_t item, uint32_t first, uint32_t last,
-                               const RenderArgs &a)
-{
-    const uint32_t lane = __lane_id();
-    uint32_t done = 0;
-    for (uint32_t c = first; c < last; c += 64u) {
-        const uint32_t i = c + lane;
-        bool want = false;
-        if (i < last) {
-            float x, y, z;
-            block_voxel(v, i, x, y, z);
-            float lam;
-            if (PREC == LYAP_PREC_PRODUCT) {
-                const ProductResult r = lambda_product_halves_w<W>(x, y, z, v.e);
-                lam = r.lam;
-                want = !(__builtin_fabsf(lam) >= v.vmargin);     /* NaN included */
-                if (v.vtau > 0.0f) {
-                    const float lo_half = r.half1 < r.half2 ? r.half1 : r.half2;
-                    want = want || (lo_half < v.vband && __builtin_fabsf(r.half1 - r.half2) > v.vtau);
-                }
-            } else {
-                lam = eval_lambda<W, PREC>(v.e, x, y, z);
-            }
-            v.vol_out[i] = lam;
-            ++done;
-        }
-        if (PREC == LYAP_PREC_PRODUCT && v.vlist_cap != 0u) {
-            const uint64_t mask = __ballot(want);
-            if (mask != 0) {
-                uint32_t base = 0;
-                if (lane == 0) base = atomicAdd(a.vox_counts + item * kHeadStride, (uint32_t)__popcll(mask));
-                base = uniform((uint32_t)__shfl((int)base, 0));
-                if (want) {
-                    const uint32_t slot = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-                    if (slot < v.vlist_cap) a.vox_list[v.vlist_base + slot] = i;
-                }
-            }
-        }
-    }
-    return done;
-}
-
 /* Three waves per SIMD (at most 168 VGPRs): the 16-slot FP32 kernels fit
  * without spilling; the 32-slot, FP64 and margin kernels would otherwise
  * take 200+ VGPRs and run two waves, and measure 20-30% slower that way than
@@ -928,15 +864,6 @@ void render_persistent(const ViewDesc *__restrict__ views, RenderArgs a)
                     if (sh_count) {
                         shade_list(views[uniform(cur_view)], sh, sh_count);
                         sh_count = 0;
-                    }
-                    if (uniform(views[tv].kind) == kItemVolume) {
-                        /* a tile of a volume block: every lane is idle, so the
-                         * wave evaluates its voxels and claims again */
-                        const unsigned long long s0 = a.wave_log ? clock64() : 0ull;
-                        done_evals += voxel_tile<W, PREC>(views[tv], tv, f, l, a);
-                        if (a.wave_log) c_eval += clock64() - s0;
-                        cur_view = 0xFFFFFFFFu;
-                        continue;
                     }
                     cur_view = tv;
                     pos = f;
@@ -1227,591 +1154,10 @@ void render_persistent(const ViewDesc *__restrict__ views, RenderArgs a)
     }
 }
 
-/* ---- march passes ------------------------------------------------------- */
-
-/* A small frame has fewer rays that meet the box than the chip has lanes, so
- * its march speculates: K lanes of a ray evaluate the next K samples at once.
- * In the persistent launch the waves also carry the refill, hand-over and
- * shading state, which holds them to three per SIMD. March passes split the
- * march instead into launches of one round each: march_pass gives each ray
- * K lanes for one round (K samples, the persistent launch's sample
- * positions, evaluation and combine) and lists the rays still marching for
- * the next pass, K rising from pass to pass as the list shrinks; ray_start
- * sets up the pixels' rays (one lane each) beforehand and lists those that
- * meet the box, and the last pass runs its rays to the end of their march.
- * Rays whose march ended park for the refinement launch as before. A ray's
- * arithmetic is the same in every schedule, so the bytes are too. (Setting
- * the rays up in the first pass instead, every lane of a group the same ray,
- * raised the pass kernel's registers and made the frame 8 % slower.) */
-
-/* A marching ray between passes (64 bytes). The passes refine by bisection,
- * where a ray's position is always C + V t, its step Fdt or Fdt /
- * nearMultiplier by the near flag, and both were formed by those same
- * expressions: the record keeps t and Fdt and the resumed ray recomputes P,
- * Ndt and dt bit for bit. */
-struct alignas(16) PassRec {
-    uint32_t pix, evals;
-    uint32_t index_flags;              /* march sample index (< 2^24), flags in the top byte */
-    uint32_t m;
-    float Vx, Vy, Vz, t, t1, Fdt, last_step, a, c, l, tb, dtb;
-};
-static_assert(sizeof(PassRec) == 64, "pass record size");
-
-__device__ __forceinline__ void store_pass(const Ray &r, PassRec &q)
-{
-    q.pix = r.pix;
-    q.evals = r.evals;
-    q.index_flags = (r.index & 0x00FFFFFFu) | (r.flags << 24);
-    q.m = r.m;
-    q.Vx = r.V.x; q.Vy = r.V.y; q.Vz = r.V.z;
-    q.t = r.t; q.t1 = r.t1; q.Fdt = r.Fdt; q.last_step = r.last_step;
-    q.a = r.a; q.c = r.c; q.l = r.l;
-    q.tb = r.tb; q.dtb = r.dtb;
-}
-
-__device__ __forceinline__ void load_pass(const ViewDesc &v, const PassRec &q, Ray &r)
-{
-    r.pix = q.pix;
-    r.evals = q.evals;
-    r.index = q.index_flags & 0x00FFFFFFu;
-    r.flags = q.index_flags >> 24;
-    r.m = q.m;
-    r.V = {q.Vx, q.Vy, q.Vz};
-    r.t = q.t; r.t1 = q.t1; r.Fdt = q.Fdt; r.last_step = q.last_step;
-    r.a = q.a; r.c = q.c; r.l = q.l;
-    r.tb = q.tb; r.dtb = q.dtb;
-    r.Ndt = r.Fdt / v.prm.nearMultiplier;          /* start_hit's expression */
-    r.dt = (r.flags & 1u) ? r.Ndt : r.Fdt;
-    r.P = add(f3(v.cam.C), mul(r.V, r.t));          /* march_step's expression */
-    r.k = 0;
-    r.launch_samples = 0;
-    r.phase = PH_MARCH;
-}
-
-struct PassArgs {
-    uint32_t n_views;
-    uint32_t K;                        /* lanes (samples) per ray in this pass */
-    const PassRec *cont_in;            /* march_pass: the rays to advance */
-    const uint32_t *in_counts;         /* per view and sub-list, kHeadStride words apart */
-    PassRec *cont_out;                 /* the rays still marching */
-    uint32_t *out_counts;
-    RefineRec *refine_out;
-    uint32_t *refine_counts;           /* per view and sub-region, kHeadStride words apart */
-    unsigned long long *eval_counter;
-    uint32_t rounds;                   /* rounds per ray (0: until the march ends) */
-};
-
-/* One wave's samples of a round (one per lane). */
-struct PassStash {
-    float lam[64], t[64], x[64], y[64], z[64];
-    uint32_t ok[64];
-    float ca[64], aa[64];
-};
-
-/* Listed rays of view v's sub-list s. */
-__device__ __forceinline__ uint32_t cont_count(const ViewDesc *__restrict__ views, const uint32_t *counts,
-                                               uint32_t v, uint32_t s)
-{
-    return uniform(min(counts[(v * kContSubs + s) * kHeadStride], views[uniform(v)].cont_cap / kContSubs));
-}
-
-/* Appends the rays of this wave's lanes with `want` (leaders) to view vi's
- * sub-list of this block's XCD (block index modulo kContSubs), one atomic
- * per wave; rays that do not fit go on to the next sub-list. A view's
- * sub-lists hold all its rays together, and a full sub-list has every one of
- * its slots written, so each ray finds a slot within kContSubs tries. */
-__device__ __forceinline__ void append_cont(const ViewDesc &v, uint32_t vi, const Ray &r, bool want,
-                                            PassRec *out, uint32_t *counts, uint32_t first = 0)
-{
-    const uint32_t lane = __lane_id();
-    const uint32_t sub_cap = v.cont_cap / kContSubs;
-    for (uint32_t tries = first; tries < kContSubs && __ballot(want) != 0; ++tries) {
-        const uint64_t m = __ballot(want);
-        const uint32_t sub = (blockIdx.x + tries) % kContSubs;
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(counts + (vi * kContSubs + sub) * kHeadStride, (uint32_t)__popcll(m));
-        base = uniform((uint32_t)__shfl((int)base, 0));
-        if (want) {
-            const uint32_t slot = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            if (slot < sub_cap) {
-                PassRec q;
-                store_pass(r, q);
-                out[v.cont_base + sub * sub_cap + slot] = q;
-                want = false;
-            }
-        }
-    }
-}
-
-/* Parks the rays of this wave's lanes with `want` (leaders) in view vi's
- * refinement records: the sub-region of this block's XCD, the next ones while
- * a sub-region is full (the regions hold twice the view's rays, so one has
- * room). One atomic per wave and try. */
-__device__ __forceinline__ RefineRec refine_record(const Ray &r)
-{
-    RefineRec q;
-    q.pix = r.pix;
-    q.evals = r.evals;
-    q.Vx = r.V.x;
-    q.Vy = r.V.y;
-    q.Vz = r.V.z;
-    q.lo = r.lo();
-    q.hi = r.hi();
-    q.l_hi = r.l_hi();
-    q.dt = r.dt;
-    q.a = r.a;
-    q.c = r.c;
-    q.l_lo = r.l_lo();
-    return q;
-}
-
-__device__ __forceinline__ void append_refine(const ViewDesc &v, uint32_t vi, const Ray &r, bool want,
-                                              RefineRec *out, uint32_t *counts, uint32_t first = 0)
-{
-    const uint32_t lane = __lane_id();
-    for (uint32_t tries = first; tries < kRefineSubs && __ballot(want) != 0; ++tries) {
-        const uint64_t m = __ballot(want);
-        const uint32_t sub = (blockIdx.x + tries) % kRefineSubs;
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(counts + (vi * kRefineSubs + sub) * kHeadStride, (uint32_t)__popcll(m));
-        base = uniform((uint32_t)__shfl((int)base, 0));
-        if (want) {
-            const uint32_t slot = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            if (slot < v.refine_cap) {
-                out[v.refine_base + sub * v.refine_cap + slot] = refine_record(r);
-                want = false;
-            }
-        }
-    }
-}
-
-/* A block's four waves append together: device-scope atomics on one address
- * take about 20 ns each, one after the other, and the 10,000 waves of a
- * 512 x 512 frame's first pass share eight addresses (39 us with an atomic
- * per wave and list, 34 us with one per block). Per wave the view and the
- * rays to list and to park; the first wave of each view present takes the
- * reservations for all of that view's waves. */
-struct BlockAppend {
-    uint32_t view[4], n_cont[4], n_refine[4];
-    uint32_t cont_base[4], refine_base[4];
-};
-
-/* Every wave of the block calls this (a wave without rays with no bits in
- * either mask). Rays that do not fit go on to the next sub-lists. */
-__device__ __forceinline__ void append_block(BlockAppend &s, const ViewDesc &v, uint32_t vi, const Ray &r,
-                                             bool cont, bool park, const PassArgs &a)
-{
-    const uint32_t lane = __lane_id();
-    const uint32_t w = threadIdx.x >> 6;
-    const uint64_t cm = __ballot(cont), pm = __ballot(park);
-    if (lane == 0) {
-        s.view[w] = vi;
-        s.n_cont[w] = (uint32_t)__popcll(cm);
-        s.n_refine[w] = (uint32_t)__popcll(pm);
-    }
-    __syncthreads();
-    /* lane 0 of a view's first wave reserves list entries, lane 1 records */
-    uint32_t first = w, before_c = 0, before_p = 0, total_c = 0, total_p = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < 4u; ++k) {
-        if (s.view[k] != vi) continue;
-        if (k < first) first = k;
-        if (k < w) {
-            before_c += s.n_cont[k];
-            before_p += s.n_refine[k];
-        }
-        total_c += s.n_cont[k];
-        total_p += s.n_refine[k];
-    }
-    if (w == first) {
-        if (lane == 0 && total_c)
-            s.cont_base[w] = atomicAdd(a.out_counts + (vi * kContSubs + blockIdx.x % kContSubs) * kHeadStride, total_c);
-        if (lane == 1 && total_p)
-            s.refine_base[w] =
-                atomicAdd(a.refine_counts + (vi * kRefineSubs + blockIdx.x % kRefineSubs) * kHeadStride, total_p);
-    }
-    __syncthreads();
-    const uint64_t below = (1ull << lane) - 1ull;
-    if (cont) {
-        const uint32_t sub_cap = v.cont_cap / kContSubs;
-        const uint32_t slot = s.cont_base[first] + before_c + (uint32_t)__popcll(cm & below);
-        if (slot < sub_cap) {
-            PassRec q;
-            store_pass(r, q);
-            a.cont_out[v.cont_base + (blockIdx.x % kContSubs) * sub_cap + slot] = q;
-            cont = false;
-        }
-    }
-    if (park) {
-        const uint32_t slot = s.refine_base[first] + before_p + (uint32_t)__popcll(pm & below);
-        if (slot < v.refine_cap) {
-            a.refine_out[v.refine_base + (blockIdx.x % kRefineSubs) * v.refine_cap + slot] = refine_record(r);
-            park = false;
-        }
-    }
-    append_cont(v, vi, r, cont, a.cont_out, a.out_counts, 1u);
-    append_refine(v, vi, r, park, a.refine_out, a.refine_counts, 1u);
-}
-
-/* Every pixel ray of every view, one lane each (a block's 256 rays belong
- * to one view: views start at multiples of 256 in this grid): misses of the
- * box are written, the others listed for the first pass with one atomic per
- * block on the sub-list of its XCD (rays that do not fit go on to the next
- * sub-lists, as append_cont). */
-__global__ __launch_bounds__(256) void ray_start(const ViewDesc *__restrict__ views, PassArgs a)
-{
-    __shared__ uint32_t wave_hits[4];
-    __shared__ uint32_t block_base;
-    const uint32_t g = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t gb = uniform(blockIdx.x * 256u);
-    uint32_t vi = 0;
-    while (vi + 1u < a.n_views && views[uniform(vi + 1u)].ray_base <= gb) ++vi;
-    vi = uniform(vi);
-    const ViewDesc &v = views[vi];
-    if (v.kind != kItemView || gb >= v.ray_base + v.n_rays) return;   /* the whole block */
-    const uint32_t lane = __lane_id();
-    const uint32_t w = threadIdx.x >> 6;
-    const uint32_t id = g - v.ray_base;
-    uint32_t pix = 0;
-    F3 V = {0.f, 0.f, 0.f};
-    float t0 = 0.f, t1 = 0.f;
-    const int k = id < v.n_rays ? ray_setup(v, id, pix, V, t0, t1) : RAY_PAD;
-    Ray r;
-    r.phase = PH_IDLE;
-    if (k == RAY_MISS) {
-        write_miss(v, pix, 0u);
-    } else if (k == RAY_HIT) {
-        start_hit(v, pix, V, t0, t1, r);
-    }
-    bool want = k == RAY_HIT;
-    const uint64_t m = __ballot(want);
-    if (lane == 0) wave_hits[w] = (uint32_t)__popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t total = wave_hits[0] + wave_hits[1] + wave_hits[2] + wave_hits[3];
-        block_base = total ? atomicAdd(a.out_counts + (vi * kContSubs + blockIdx.x % kContSubs) * kHeadStride,
-                                       total)
-                           : 0u;
-    }
-    __syncthreads();
-    uint32_t before = 0;
-    for (uint32_t k2 = 0; k2 < w; ++k2) before += wave_hits[k2];
-    if (want) {
-        const uint32_t sub_cap = v.cont_cap / kContSubs;
-        const uint32_t slot = block_base + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if (slot < sub_cap) {
-            PassRec q;
-            store_pass(r, q);
-            a.cont_out[v.cont_base + (blockIdx.x % kContSubs) * sub_cap + slot] = q;
-            want = false;
-        }
-    }
-    append_cont(v, vi, r, want, a.cont_out, a.out_counts);
-}
-
-/* One round for every listed ray, K lanes each (the samples of sample_point
- * ranks 0..K-1), then: rays whose march ended on a miss are written, rays
- * that found their opaque sample park for the refinement launch, the others
- * are listed for the next pass. DRAIN: `rounds` rounds (0: until the march
- * of every ray of the wave has ended) instead of one. */
-template <int W, int PREC, bool DRAIN>
-__global__ __launch_bounds__(256) void march_pass(const ViewDesc *__restrict__ views, PassArgs a)
-{
-    __shared__ PassStash stash[4];
-    __shared__ BlockAppend appends;
-    PassStash &st = stash[threadIdx.x >> 6];
-    const uint32_t lane = __lane_id();
-    const uint32_t K = uniform(a.K);
-    const uint32_t per = 64u / K;                 /* rays per wave and round */
-    const uint32_t rank = lane % K;
-    const uint32_t gbase = lane - rank;
-    const uint64_t kmask = K >= 64u ? ~0ull : ((1ull << K) - 1ull);
-    const uint32_t n_waves = gridDim.x * 4u;
-    const uint32_t wid = uniform(blockIdx.x * 4u + threadIdx.x / 64u);
-    const uint32_t pairs = a.n_views * kContSubs;
-    const bool held = pairs <= 64u;
-    ChunkMap cm{0u, 0u, 0u};
-    uint32_t chunks = 0;
-    if (held) {
-        uint32_t n = 0;
-        if (lane < pairs) n = min(a.in_counts[lane * kHeadStride], views[lane / kContSubs].cont_cap / kContSubs);
-        cm = chunk_map(n, per, lane);
-        chunks = cm.total;
-    } else {
-        for (uint32_t p = 0; p < pairs; ++p)
-            chunks += (cont_count(views, a.in_counts, p / kContSubs, p % kContSubs) + per - 1u) / per;
-    }
-    uint32_t done_evals = 0;
-    /* the four waves of a block take neighbouring chunks; the one-round
-     * passes append as a block, so a wave past the last chunk stays (without
-     * rays) while others of its block have one */
-    for (uint32_t c = wid; (DRAIN ? c : c - (wid & 3u)) < chunks; c += n_waves) {
-        uint32_t acc = 0, p = 0, cnt = 0;
-        if (!DRAIN && c >= chunks) {
-            acc = c;
-        } else if (held) {
-            chunk_find(cm, c, per, p, acc, cnt);
-        } else {
-            for (; p < pairs; ++p) {
-                cnt = cont_count(views, a.in_counts, p / kContSubs, p % kContSubs);
-                const uint32_t nc = (cnt + per - 1u) / per;
-                if (c < acc + nc) break;
-                acc += nc;
-            }
-        }
-        const uint32_t vi = uniform(p / kContSubs);
-        const ViewDesc &v = views[vi];
-        const uint32_t i = (c - acc) * per + lane / K;
-        bool busy = i < cnt;
-        Ray r;
-        r.phase = PH_IDLE;
-        if (busy) load_pass(v, a.cont_in[v.cont_base + (p % kContSubs) * (v.cont_cap / kContSubs) + i], r);
-        /* `rounds` rounds (0: until every ray of the wave has ended); a ray
-         * whose march ends leaves its group idle */
-        for (uint32_t round = 0;; ++round) {
-            float lam = NAN;
-            F3 sp = {0.f, 0.f, 0.f};
-            float ts = 0.f;
-            const bool valid = busy && sample_point(v, r, rank, K, sp, ts);
-            if (valid) lam = eval_lambda<W, PREC>(v.e, sp.x, sp.y, sp.z);
-            /* does sample `rank` stop the march (opaque, invalid, a near/far
-             * toggle, or jitter, whose step needs this lambda)? */
-            bool ev = true;
-            if (valid) {
-                const LyapParams &prm = v.prm;
-                const bool near_ = (r.flags & 1u) != 0;
-                const bool toggles = (r.index + rank) > 0 && r.Ndt != r.Fdt &&
-                                     ((lam <= prm.nearThreshold) != near_);
-                ev = !(lam > prm.opaqueThreshold) || toggles || prm.jitter != 0.0f;
-            }
-            const uint64_t evm = (__ballot(ev) >> gbase) & kmask;
-            /* the previous round's combine has read the stash */
-            wave_sync_lds();
-            st.lam[lane] = lam;
-            st.t[lane] = ts;
-            st.x[lane] = sp.x;
-            st.y[lane] = sp.y;
-            st.z[lane] = sp.z;
-            st.ok[lane] = valid ? 1u : 0u;
-            float sc = 0.0f, sa = 0.0f;
-            if (busy && r.index + rank > 0u) {
-                if (lam > v.prm.chaosThreshold) sc = lam;
-                else if (lam > v.prm.opaqueThreshold) sa = lam;
-            }
-            st.ca[lane] = sc;
-            st.aa[lane] = sa;
-            wave_sync_lds();
-            bool finished = false;
-            combine_march<PassStash, 64u>(v, r, evm, st, gbase, K, busy ? (int)PH_MARCH : (int)PH_IDLE,
-                                          rank == 0, finished);
-            if (finished && rank == 0) done_evals += r.evals;
-            const bool park = busy && rank == 0 && r.phase == PH_REFINE;
-            busy = busy && r.phase == PH_MARCH;
-            if (!DRAIN) {
-                append_block(appends, v, vi, r, busy && rank == 0, park, a);
-                break;
-            }
-            append_refine(v, vi, r, park, a.refine_out, a.refine_counts);
-            if ((a.rounds != 0 && round + 1u >= a.rounds) || __ballot(busy) == 0) break;
-        }
-        if (DRAIN) append_cont(v, vi, r, busy && rank == 0, a.cont_out, a.out_counts);
-    }
-    count_evals(a.eval_counter, done_evals, wid);
-}
-
-/* ---- refinement launch -------------------------------------------------- */
-
-struct RefineArgs {
-    uint32_t n_views;
-    const RefineRec *recs;
-    const uint32_t *counts;            /* per view and sub-region, kHeadStride words apart */
-    unsigned long long *eval_counter;
-};
-
-/* Records of view-sub-region pair p that the march launches wrote. */
-__device__ __forceinline__ uint32_t refine_count(const ViewDesc *__restrict__ views,
-                                                 const RefineArgs &a, uint32_t p)
-{
-    return uniform(min(a.counts[p * kHeadStride], views[uniform(p / kRefineSubs)].refine_cap));
-}
-
-/* Finishes the parked rays, two lanes per ray and 32 rays of one view per
- * wave: the bisection of [lo, hi] (the midpoint rule), the six normal
- * samples in the order x-, x+, y-, y+, z-, z+ (kernel.cu:456-473), the hit
- * record and its colour. Per bisection trip the first lane evaluates the
- * midpoint and the second the midpoint of the half the crossing of the
- * line through lambda at lo and hi falls in; when that half is the one the
- * first sample chooses, the trip resolves two levels. The normal takes three
- * trips, the minus samples on the first lane and the plus samples on the
- * second. The arithmetic is the march kernel's, step for step, so the bytes
- * are those of refining in place. */
-template <int W, int PREC, bool MARGIN>
-__device__ __forceinline__ float refine_eval(const ViewDesc &v, F3 sp, float thr)
-{
-    float lam = eval_lambda<W, PREC>(v.e, sp.x, sp.y, sp.z);
-    if (MARGIN && PREC != LYAP_PREC_FP64 && !(__builtin_fabsf(lam - thr) >= v.margin))
-        lam = eval_fp64_call<W>(v.e, sp.x, sp.y, sp.z);
-    return lam;
-}
-
-template <int W, int PREC, bool MARGIN>
-__global__ __launch_bounds__(256) void refine_rays(const ViewDesc *__restrict__ views, RefineArgs a)
-{
-    const uint32_t lane = __lane_id();
-    const uint32_t side = lane & 1u;           /* 0: midpoints, minus normal samples */
-    const uint32_t n_waves = gridDim.x * 4u;
-    const uint32_t wid = uniform(blockIdx.x * 4u + threadIdx.x / 64u);
-    const uint32_t pairs = a.n_views * kRefineSubs;
-    const bool held = pairs <= 64u;
-    ChunkMap cm{0u, 0u, 0u};
-    uint32_t total = 0;
-    if (held) {
-        uint32_t n = 0;
-        if (lane < pairs) n = min(a.counts[lane * kHeadStride], views[lane / kRefineSubs].refine_cap);
-        cm = chunk_map(n, 32u, lane);
-        total = cm.total;
-    } else {
-        for (uint32_t p = 0; p < pairs; ++p) total += (refine_count(views, a, p) + 31u) / 32u;
-    }
-    unsigned long long done = 0;
-    for (uint32_t t = wid; t < total; t += n_waves) {
-        uint32_t acc = 0, p = 0, n = 0;
-        if (held) {
-            chunk_find(cm, t, 32u, p, acc, n);
-        } else {
-            for (; p < pairs; ++p) {
-                n = refine_count(views, a, p);
-                const uint32_t nt = (n + 31u) / 32u;
-                if (t < acc + nt) break;
-                acc += nt;
-            }
-        }
-        const ViewDesc &v = views[uniform(p / kRefineSubs)];
-        const uint32_t i = (t - acc) * 32u + (lane >> 1);
-        const bool has = i < n;
-        RefineRec q{};
-        if (has) q = a.recs[v.refine_base + (p % kRefineSubs) * v.refine_cap + i];
-        const F3 C = f3(v.cam.C);
-        const F3 V = {q.Vx, q.Vy, q.Vz};
-        const float thr = v.prm.opaqueThreshold;
-        float lo = q.lo, hi = q.hi, l_hi = q.l_hi, l_lo = q.l_lo;
-        uint32_t evals = q.evals;
-        /* both lanes of a ray hold the same interval; trips are wave-uniform */
-        for (int k = 0; __ballot(has && k < v.bisect_steps) != 0;) {
-            const bool go = has && k < v.bisect_steps;
-            const float mid = lo + (hi - lo) * 0.5f;
-            /* the half the line's crossing falls in, and its midpoint */
-            const float f = (l_lo - thr) / (l_lo - l_hi);
-            const bool guess_lo = !(lo + (hi - lo) * f > mid);
-            const float mid2 = guess_lo ? lo + (mid - lo) * 0.5f : mid + (hi - mid) * 0.5f;
-            float lam = 0.f;
-            if (go) lam = refine_eval<W, PREC, MARGIN>(v, add(C, mul(V, side ? mid2 : mid)), thr);
-            const float lm = __shfl(lam, (int)(lane & ~1u));
-            const float lg = __shfl(lam, (int)(lane | 1u));
-            if (go) {
-                ++evals;
-                ++k;
-                const bool opaque = !(lm > thr);
-                if (opaque) { hi = mid; l_hi = lm; }
-                else { lo = mid; l_lo = lm; }
-                if (k < v.bisect_steps && opaque == guess_lo) {
-                    /* the guessed half is the one taken: its midpoint, formed
-                     * from the same interval, is the next level's */
-                    ++evals;
-                    ++k;
-                    const float m2 = lo + (hi - lo) * 0.5f;
-                    if (!(lg > thr)) { hi = m2; l_hi = lg; }
-                    else { lo = m2; l_lo = lg; }
-                }
-            }
-        }
-        Ray r;
-        r.pix = q.pix;
-        r.t = hi;
-        r.P = add(C, mul(V, hi));
-        r.l = l_hi;
-        r.a = q.a;
-        r.c = q.c;
-        const float h = (v.normal_h > 0.0f) ? v.normal_h : q.dt * v.prm.gradient;
-        float g[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-        for (uint32_t ax = 0; ax < 3u; ++ax) {
-            F3 sp = r.P;
-            const float off = side ? h : -h;
-            if (ax == 0) sp.x = r.P.x + off;
-            else if (ax == 1) sp.y = r.P.y + off;
-            else sp.z = r.P.z + off;
-            float lam = 0.f;
-            if (has) lam = eval_lambda<W, PREC>(v.e, sp.x, sp.y, sp.z);
-            const float lminus = __shfl(lam, (int)(lane & ~1u));
-            const float lplus = __shfl(lam, (int)(lane | 1u));
-            g[ax] = -lminus;
-            g[ax] = g[ax] + lplus;
-        }
-        if (has && side == 0) {
-            r.evals = evals + 6u;
-            const F3 N = normalized({g[0], g[1], g[2]});
-            write_hit(v, r.pix, r.evals, r.P, N, r.t, r.l, r.a, r.c);
-            const C4 cc = shade(r.P, N, r.a, r.c, v.cam, v.lights, v.num_lights);
-            LyapRGBA px;
-            px.r = to_u8(cc.x);
-            px.g = to_u8(cc.y);
-            px.b = to_u8(cc.z);
-            px.a = to_u8(cc.w);
-            v.rgba[r.pix] = px;
-            done += evals + 6u;
-        }
-    }
-    count_evals(a.eval_counter, done, wid);
-}
-/* ---- FP64 pass over the volume blocks' lists ---------------------------- */
-
-struct VoxelFp64Args {
-    uint32_t n_items;
-    const uint32_t *list;
-    const uint32_t *counts;            /* per item, kHeadStride words apart */
-};
-
-__device__ __forceinline__ uint32_t listed(const ViewDesc *__restrict__ views,
-                                           const VoxelFp64Args &a, uint32_t p)
-{
-    return uniform(min(a.counts[p * kHeadStride], views[uniform(p)].vlist_cap));
-}
-
-/* Re-evaluates the listed voxels of every volume block in FP64 (the same
- * lambda_fp64 arithmetic as the volume kernels' FP64 pass), 64 entries of
- * one block per wave. */
-template <int W>
-__global__ __launch_bounds__(256) void voxel_fp64(const ViewDesc *__restrict__ views, VoxelFp64Args a)
-{
-    const uint32_t lane = __lane_id();
-    const uint32_t n_waves = gridDim.x * 4u;
-    const uint32_t wid = uniform(blockIdx.x * 4u + threadIdx.x / 64u);
-    uint32_t total = 0;
-    for (uint32_t p = 0; p < a.n_items; ++p) total += (listed(views, a, p) + 63u) / 64u;
-    for (uint32_t t = wid; t < total; t += n_waves) {
-        uint32_t acc = 0, p = 0, n = 0;
-        for (; p < a.n_items; ++p) {
-            n = listed(views, a, p);
-            const uint32_t nt = (n + 63u) / 64u;
-            if (t < acc + nt) break;
-            acc += nt;
-        }
-        const ViewDesc &v = views[uniform(p)];
-        const uint32_t j = (t - acc) * 64u + lane;
-        if (j < n) {
-            const uint32_t i = a.list[v.vlist_base + j];
-            float x, y, z;
-            block_voxel(v, i, x, y, z);
-            v.vol_out[i] = (float)lambda_fp64_w<W>(x, y, z, v.e);
-        }
-    }
-}
-
-/* Up to four word arrays cleared by one launch: blockIdx.y picks the array. */
+/* Up to three word arrays cleared by one launch: blockIdx.y picks the array. */
 struct ZeroRegions {
-    uint32_t *p[4];
-    uint32_t n[4];
+    uint32_t *p[3];
+    uint32_t n[3];
 };
 
 __global__ void zero_regions(ZeroRegions z)
@@ -1850,35 +1196,6 @@ static void fill_view(ViewDesc &v, const EvalDesc &e, const LyapCam &cam,
     v.normal_h = mode.normal_h;
     v.margin = mode.fp64_margin;
     v.max_samples = 1u << 20;
-    v.kind = kItemView;
-}
-
-/* Fills a volume-block item: z slices [z_begin, z_end) of the nx*ny*nz grid
- * over [lo, hi) with output `out` (slice z_begin), under `mode`'s rule. */
-static void fill_block(ViewDesc &v, const EvalDesc &e, const LyapParams &prm, const float lo[3],
-                       const float hi[3], const uint32_t n[3], uint32_t z_begin, uint32_t z_end,
-                       float *out, const LyapVolumeMode &mode)
-{
-    std::memset(&v, 0, sizeof(v));
-    v.kind = kItemVolume;
-    v.e = e;
-    v.prm = prm;
-    v.vol_out = out;
-    v.vnx = n[0];
-    v.vny = n[1];
-    v.vnz = n[2];
-    v.vz0 = z_begin;
-    for (int k = 0; k < 3; ++k) {
-        v.vlo[k] = lo[k];
-        v.vspan[k] = hi[k] - lo[k];
-    }
-    v.n_rays = n[0] * n[1] * (z_end - z_begin);
-    const bool reeval = mode.precision == LYAP_PREC_PRODUCT &&
-                        (mode.fp64_margin > 0.0f || mode.converge_tau > 0.0f);
-    v.vmargin = reeval ? mode.fp64_margin : 0.0f;
-    v.vtau = reeval ? mode.converge_tau : 0.0f;
-    v.vband = mode.converge_band;
-    v.vlist_cap = reeval ? v.n_rays : 0u;
 }
 
 /* ---- launch planning ----------------------------------------------------- */
@@ -1901,15 +1218,12 @@ static uint32_t default_lanes_per_ray(uint32_t resident_lanes, uint64_t rays)
  * claims are many times the number of waves and the queue balances. */
 struct LaunchPlan {
     uint32_t blocks, lanes_per_ray, tile_rays, resident_lanes, slots;
-    uint32_t voxel_tile;          /* voxels per claim of a volume block */
     uint32_t budget[3];           /* level budgets chosen by the tuning, 0 = built-in */
     bool direct;
     bool levels;                  /* the persistent levels only: no march passes */
+    bool shaped;                  /* a shape of the persistent levels was asked for */
+    MarchPlan march;              /* n 0: the persistent levels (set by prepare_views) */
 };
-
-/* Voxels per work-queue claim of a volume block unless tuned: four waves'
- * worth, so claims are cheap next to the evaluations they hand out. */
-static const uint32_t kDefaultVoxelTile = 256u;
 
 /* Samples each lane evaluates per round unless tuned. More than one halves
  * the lanes a ray's control work is replicated on, but measured on the
@@ -1990,8 +1304,9 @@ static LaunchPlan plan_launch(const lyap_ctx *ctx, uint64_t rays, const LyapTuni
     if (p.lanes_per_ray * p.slots > 64u) p.lanes_per_ray = 64u / p.slots;
     p.tile_rays = tune.tile_rays ? tune.tile_rays : 64u / p.lanes_per_ray;
     if (p.tile_rays == 0) p.tile_rays = 1;
-    p.voxel_tile = tune.voxel_tile ? (tune.voxel_tile + 63u) / 64u * 64u : kDefaultVoxelTile;
     for (int k = 0; k < 3; ++k) p.budget[k] = tune.level_budget[k];
+    p.shaped = tune.lanes_per_ray || tune.slots || tune.level_budget[0] || tune.level_budget[1] ||
+               tune.level_budget[2];
     if (direct) {
         p.lanes_per_ray = 1;
         p.slots = 1;
@@ -2029,10 +1344,6 @@ struct RenderResources {
     size_t refine_buf_bytes = 0;
     void *refine_counts = nullptr;   /* per view and sub-region, one 128 B line each */
     size_t refine_counts_bytes = 0;
-    void *vox_list = nullptr;        /* volume blocks' FP64 re-evaluation lists */
-    size_t vox_list_bytes = 0;
-    void *vox_counts = nullptr;      /* per item, one 128 B line each */
-    size_t vox_counts_bytes = 0;
 };
 
 static int ensure_buffer(lyap_ctx *ctx, void **buf, size_t *cap, size_t bytes, bool may_sync)
@@ -2055,8 +1366,6 @@ static void release_resources(lyap_ctx *ctx, RenderResources &r)
     ctx_free(ctx, r.cont_counts);
     ctx_free(ctx, r.refine_buf);
     ctx_free(ctx, r.refine_counts);
-    ctx_free(ctx, r.vox_list);
-    ctx_free(ctx, r.vox_counts);
     ctx_free(ctx, r.counters);
     for (int k = 0; k < 2; ++k) {
         if (r.staging[k]) (void)hipHostFree(r.staging[k]);
@@ -2070,98 +1379,50 @@ static void release_resources(lyap_ctx *ctx, RenderResources &r)
  * reference's launch shape keeps every ray on its lane). */
 static bool parks(const LaunchPlan &plan, const ViewDesc *views)
 {
-    /* views come before volume blocks in a launch's table */
-    return !plan.direct && views[0].kind == kItemView && views[0].refine == LYAP_REFINE_BISECT &&
+    return !plan.direct && views[0].refine == LYAP_REFINE_BISECT &&
            views[0].bisect_steps > 0;
 }
 
-/* Whether the launch runs in walk_rays: every item a view refined by the
- * walk whose step jitter keeps its samples from being taken ahead. */
+/* Whether the launch runs in walk_rays: every view refined by the walk, its
+ * jitter keeping its samples from being taken ahead. */
 static bool walks(const LaunchPlan &plan, const ViewDesc *views, unsigned n_views)
 {
     if (plan.direct || plan.levels) return false;
     for (unsigned i = 0; i < n_views; ++i)
-        if (views[i].kind != kItemView || views[i].refine != LYAP_REFINE_WALK || views[i].prm.jitter == 0.0f)
+        if (views[i].refine != LYAP_REFINE_WALK || views[i].prm.jitter == 0.0f)
             return false;
     return n_views > 0;
 }
 
-/* March passes (march_pass): the lanes per ray of each pass, at most
- * kMaxPasses of them; rays still marching after the last pass finish in a
- * persistent launch. */
-constexpr uint32_t kMaxPasses = 12;
+/* Entries of each of `subs` sub-lists that hold `rays` rays together. */
+static uint32_t pass_cap(uint32_t rays, uint32_t subs) { return (rays + subs - 1u) / subs; }
 
-struct PassPlan {
-    uint32_t n = 0;                   /* passes; 0: the persistent levels */
-    uint32_t K[kMaxPasses] = {};
-    uint32_t R[kMaxPasses] = {};      /* rounds of each pass (0: until the rays end) */
-};
-
-/* March passes for small launches of views refined by bisection (the
- * batched schedule's plan gives four or more lanes per ray): K = 4, 8, 16,
- * 32, 64, 64 lanes per ray for one round each, then 64 lanes until the rays
- * end. Measured on the 512x512 frame against other sequences: starting at 8
- * lanes, fewer or more 64-lane passes, or no draining pass (a persistent
- * launch finishing the rays) were 1-12 % slower. LYAP_MARCH_PASSES
- * overrides the sequence ("K" or "KxR" per pass, R rounds, 0 = until the
- * rays end; "0" switches the passes off). */
-static PassPlan pass_plan(const LaunchPlan &plan, const ViewDesc *views, unsigned n_views)
+/* The march passes, for a launch of up to 64 views refined by bisection unless
+ * a shape of the persistent levels was asked for. Their lists take 144 bytes a
+ * ray, as the levels' do. */
+static MarchPlan choose_march(const LaunchPlan &plan, const ViewDesc *views, unsigned n_views)
 {
-    PassPlan pp;
-    /* a pass finds each chunk's view and sub-list by a scan over them, so
-     * launches of many views keep the persistent levels */
-    if (plan.direct || plan.levels || !parks(plan, views) || plan.lanes_per_ray < 4u || n_views > 16u)
-        return pp;
-    for (unsigned i = 0; i < n_views; ++i)
-        if (views[i].kind != kItemView) return pp;
-    /* "K" or "KxR" per pass, comma separated */
-    static const char *env = std::getenv("LYAP_MARCH_PASSES");
-    const char *c = env ? env : "4,8,16,32,64,64,64x0";
-    /* (the last pass always runs its rays to the end: its records are the
-     * passes' own, which the persistent launches do not read) */
-    if (c[0] == '0' && c[1] == 0) return pp;
-    while (*c && pp.n < kMaxPasses) {
-        char *e = nullptr;
-        const unsigned long k = std::strtoul(c, &e, 10);
-        if (k == 0 || k > 64 || (k & (k - 1))) return PassPlan{};
-        unsigned long r = 1;
-        if (*e == 'x') r = std::strtoul(e + 1, &e, 10);
-        pp.K[pp.n] = (uint32_t)k;
-        pp.R[pp.n] = (uint32_t)r;
-        ++pp.n;
-        if (*e != ',') break;
-        c = e + 1;
-    }
-    if (pp.n) pp.R[pp.n - 1] = 0;
-    return pp;
+    if (plan.direct || plan.levels || plan.shaped || !parks(plan, views)) return MarchPlan{};
+    uint64_t rays = 0;
+    for (unsigned i = 0; i < n_views; ++i) rays += views[i].n_rays;
+    return march_plan(n_views, rays);
 }
 
 /* Prepares `views` for a launch: tile ranges, continuation regions, the
  * common coefficient window; sizes the resources and fills the pinned
  * staging copy. `may_sync` is false while a stream capture is open. */
 static int prepare_views(lyap_ctx *ctx, RenderResources &res, ViewDesc *views,
-                         unsigned n_views, const LaunchPlan &plan, uint32_t W,
+                         unsigned n_views, LaunchPlan &plan, uint32_t W,
                          bool may_sync, uint32_t *total_tiles)
 {
     uint32_t tiles = 0;
-    uint64_t cap_total = 0, refine_total = 0, list_total = 0, ray_total = 0;
-    const bool passes = pass_plan(plan, views, n_views).n > 0;
+    uint64_t cap_total = 0, refine_total = 0, ray_total = 0;
+    plan.march = choose_march(plan, views, n_views);
+    const bool passes = plan.march.n > 0;
+    const uint32_t subs = passes ? plan.march.subs : kRefineSubs;
     for (unsigned i = 0; i < n_views; ++i) {
         if (views[i].e.W != W) rebuild_blocks(&views[i].e, W);
         views[i].tile_begin = tiles;
-        if (views[i].kind == kItemVolume) {
-            /* a volume block: voxel tiles, its list region, no ray buffers */
-            views[i].tile_len = plan.voxel_tile;
-            views[i].n_tiles = (views[i].n_rays + plan.voxel_tile - 1) / plan.voxel_tile;
-            tiles += views[i].n_tiles;
-            views[i].cont_base = (uint32_t)cap_total;
-            views[i].cont_cap = 0;
-            views[i].refine_base = (uint32_t)refine_total;
-            views[i].refine_cap = 0;
-            views[i].vlist_base = (uint32_t)list_total;
-            list_total += views[i].vlist_cap;
-            continue;
-        }
         views[i].tile_len = plan.tile_rays;
         views[i].n_tiles = (views[i].n_rays + plan.tile_rays - 1) / plan.tile_rays;
         tiles += views[i].n_tiles;
@@ -2169,47 +1430,43 @@ static int prepare_views(lyap_ctx *ctx, RenderResources &res, ViewDesc *views,
          * march passes list every ray that meets the box */
         uint32_t cap = views[i].n_rays / 4u;
         if (cap < 256u) cap = 256u;
-        if (passes) cap = views[i].n_rays;
-        /* ray_start's grid: every view starts a block of its own */
+        if (passes) cap = pass_cap(views[i].n_rays, subs) * subs;
+        /* a grid of one lane per ray: every view starts a block of its own */
         views[i].ray_base = (uint32_t)ray_total;
         ray_total += (views[i].n_rays + 255u) / 256u * 256u;
         views[i].cont_base = (uint32_t)cap_total;
         views[i].cont_cap = cap;
         cap_total += cap;
-        /* refinement records: each sub-region holds twice its share of the
-         * view's rays before a ray has to be refined in place (or, in the
-         * march passes, go to the next sub-region) */
+        /* refinement records: each sub-list holds twice its share of the
+         * view's rays before a ray has to be refined in place; in the march
+         * passes, where it goes to the next sub-list, its share */
         uint32_t rcap = (2u * views[i].n_rays + kRefineSubs - 1u) / kRefineSubs;
         if (rcap < 64u) rcap = 64u;
+        if (passes) rcap = pass_cap(views[i].n_rays, subs);
         views[i].refine_base = (uint32_t)refine_total;
         views[i].refine_cap = rcap;
-        refine_total += (uint64_t)rcap * kRefineSubs;
+        refine_total += (uint64_t)rcap * subs;
     }
-    if (cap_total > 0xFFFFFFFFull || refine_total > 0xFFFFFFFFull || list_total > 0xFFFFFFFFull ||
+    if (cap_total > 0xFFFFFFFFull || refine_total > 0xFFFFFFFFull ||
         ray_total > 0xFFFFFFFFull)
-        return fail(ctx, LYAP_ERR_UNSUPPORTED, "too many rays or voxels in one launch");
+        return fail(ctx, LYAP_ERR_UNSUPPORTED, "too many rays in one launch");
     *total_tiles = tiles;
     const size_t table = sizeof(ViewDesc) * n_views;
-    int rc = ensure_buffer(ctx, &res.cont_buf, &res.cont_buf_bytes, 2 * cap_total * sizeof(ContEntry), may_sync);
+    int rc = ensure_buffer(ctx, &res.cont_buf, &res.cont_buf_bytes, 2 * cap_total * (passes ? kPassRecBytes : sizeof(ContEntry)),
+                           may_sync);
     if (rc) return rc;
     rc = ensure_buffer(ctx, &res.cont_counts, &res.cont_counts_bytes,
-                       (size_t)(kMaxPasses + 1) * n_views * kContSubs * kHeadStride * sizeof(uint32_t), may_sync);
+                       passes ? (size_t)(plan.march.n + 1u) * n_views * subs * kHeadStride * sizeof(uint32_t)
+                              : (size_t)3 * n_views * sizeof(uint32_t), may_sync);
     if (rc) return rc;
     if (parks(plan, views)) {
         rc = ensure_buffer(ctx, &res.refine_buf, &res.refine_buf_bytes, refine_total * sizeof(RefineRec),
                            may_sync);
         if (rc) return rc;
         rc = ensure_buffer(ctx, &res.refine_counts, &res.refine_counts_bytes,
-                           (size_t)n_views * kRefineSubs * kHeadStride * sizeof(uint32_t), may_sync);
+                           (size_t)n_views * subs * kHeadStride * sizeof(uint32_t), may_sync);
         if (rc) return rc;
     }
-    if (list_total > 0) {
-        rc = ensure_buffer(ctx, &res.vox_list, &res.vox_list_bytes, list_total * sizeof(uint32_t), may_sync);
-        if (rc) return rc;
-    }
-    rc = ensure_buffer(ctx, &res.vox_counts, &res.vox_counts_bytes,
-                       (size_t)n_views * kHeadStride * sizeof(uint32_t), may_sync);
-    if (rc) return rc;
     rc = ensure_buffer(ctx, &res.view_table, &res.view_table_bytes, table, may_sync);
     if (rc) return rc;
     if (!res.counters) {
@@ -2236,116 +1493,6 @@ static int prepare_views(lyap_ctx *ctx, RenderResources &res, ViewDesc *views,
     return LYAP_OK;
 }
 
-/* The refinement launch over one record set, on `stream`. */
-static int launch_refine(lyap_ctx *ctx, const RenderResources &res, unsigned n_views, uint32_t W,
-                         int precision, bool margin)
-{
-    RefineArgs ra{};
-    ra.n_views = n_views;
-    ra.recs = (const RefineRec *)res.refine_buf;
-    ra.counts = (const uint32_t *)res.refine_counts;
-    ra.eval_counter = (unsigned long long *)res.counters;
-    const uint32_t cus = ctx->num_cus > 0 ? (uint32_t)ctx->num_cus : 256u;
-    const uint32_t blocks = cus * 8u;
-#define LYAP_LAUNCH(WW, PP, MM)                                                                     \
-    hipLaunchKernelGGL((refine_rays<WW, PP, MM>), dim3(blocks), dim3(256), 0, ctx->stream,          \
-                       (const ViewDesc *)res.view_table, ra)
-    if (W == 16) {
-        if (precision == LYAP_PREC_PLAIN) LYAP_LAUNCH(16, LYAP_PREC_PLAIN, false);
-        else if (precision == LYAP_PREC_PRODUCT && margin) LYAP_LAUNCH(16, LYAP_PREC_PRODUCT, true);
-        else if (precision == LYAP_PREC_PRODUCT) LYAP_LAUNCH(16, LYAP_PREC_PRODUCT, false);
-        else LYAP_LAUNCH(16, LYAP_PREC_FP64, false);
-    } else {
-        if (precision == LYAP_PREC_PLAIN) LYAP_LAUNCH(32, LYAP_PREC_PLAIN, false);
-        else if (precision == LYAP_PREC_PRODUCT && margin) LYAP_LAUNCH(32, LYAP_PREC_PRODUCT, true);
-        else if (precision == LYAP_PREC_PRODUCT) LYAP_LAUNCH(32, LYAP_PREC_PRODUCT, false);
-        else LYAP_LAUNCH(32, LYAP_PREC_FP64, false);
-    }
-#undef LYAP_LAUNCH
-    LYAP_HIP(ctx, hipGetLastError());
-    return LYAP_OK;
-}
-
-template <int W, int PREC, bool DRAIN>
-static uint32_t pass_blocks_per_cu()
-{
-    static int cached = -1;
-    if (cached < 0) {
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &n, reinterpret_cast<const void *>(&march_pass<W, PREC, DRAIN>), 256, 0) != hipSuccess ||
-            n <= 0)
-            n = 2;
-        cached = n;
-    }
-    return (uint32_t)cached;
-}
-
-/* Enqueues ray_start and the march passes: ray_start lists the pixels' rays
- * that meet the box under counts[0], pass p reads the rays listed under
- * counts[p] and lists the rays still marching under counts[p + 1] (the two
- * buffers alternate). */
-static int enqueue_passes(lyap_ctx *ctx, RenderResources &res, const ViewDesc *views, unsigned n_views,
-                          const PassPlan &pp, uint32_t W, int precision)
-{
-    uint64_t cap_total = 0, rays = 0;
-    for (unsigned i = 0; i < n_views; ++i) {
-        cap_total += views[i].cont_cap;
-        rays += (views[i].n_rays + 255u) / 256u * 256u;
-    }
-    PassRec *buf[2] = {(PassRec *)res.cont_buf, (PassRec *)res.cont_buf + cap_total};
-    uint32_t *counts = (uint32_t *)res.cont_counts;
-    const uint32_t pass_words = n_views * kContSubs * kHeadStride;
-    const uint32_t cus = ctx->num_cus > 0 ? (uint32_t)ctx->num_cus : 256u;
-    PassArgs a{};
-    a.n_views = n_views;
-    a.refine_out = (RefineRec *)res.refine_buf;
-    a.refine_counts = (uint32_t *)res.refine_counts;
-    a.eval_counter = (unsigned long long *)res.counters;
-    a.cont_out = buf[0];
-    a.out_counts = counts;
-    int rc = timing_mark(ctx);
-    if (rc) return rc;
-    hipLaunchKernelGGL(ray_start, dim3((uint32_t)((rays + 255u) / 256u)), dim3(256), 0, ctx->stream,
-                       (const ViewDesc *)res.view_table, a);
-    LYAP_HIP(ctx, hipGetLastError());
-    rc = timing_mark(ctx);
-    if (rc) return rc;
-    for (uint32_t p = 0; p < pp.n; ++p) {
-        a.K = pp.K[p];
-        a.rounds = pp.R[p];
-        a.cont_in = buf[p & 1u];
-        a.in_counts = counts + p * pass_words;
-        a.cont_out = buf[(p + 1u) & 1u];
-        a.out_counts = counts + (p + 1u) * pass_words;
-        rc = timing_mark(ctx);
-        if (rc) return rc;
-#define LYAP_LAUNCH(WW, PP, DD)                                                                      \
-    hipLaunchKernelGGL((march_pass<WW, PP, DD>), dim3(cus * pass_blocks_per_cu<WW, PP, DD>()), dim3(256), \
-                       0, ctx->stream, (const ViewDesc *)res.view_table, a)
-#define LYAP_LAUNCH2(WW, PP)                                                                         \
-    do {                                                                                             \
-        if (a.rounds == 1u) LYAP_LAUNCH(WW, PP, false);                                              \
-        else LYAP_LAUNCH(WW, PP, true);                                                              \
-    } while (0)
-        if (W == 16) {
-            if (precision == LYAP_PREC_PLAIN) LYAP_LAUNCH2(16, LYAP_PREC_PLAIN);
-            else if (precision == LYAP_PREC_PRODUCT) LYAP_LAUNCH2(16, LYAP_PREC_PRODUCT);
-            else LYAP_LAUNCH2(16, LYAP_PREC_FP64);
-        } else {
-            if (precision == LYAP_PREC_PLAIN) LYAP_LAUNCH2(32, LYAP_PREC_PLAIN);
-            else if (precision == LYAP_PREC_PRODUCT) LYAP_LAUNCH2(32, LYAP_PREC_PRODUCT);
-            else LYAP_LAUNCH2(32, LYAP_PREC_FP64);
-        }
-#undef LYAP_LAUNCH2
-#undef LYAP_LAUNCH
-        LYAP_HIP(ctx, hipGetLastError());
-        rc = timing_mark(ctx);
-        if (rc) return rc;
-    }
-    return LYAP_OK;
-}
-
 /* Enqueues the upload and the level launches on the context's stream. No
  * call here synchronises, so it may be recorded into a graph. */
 static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *views,
@@ -2360,28 +1507,22 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
     ZeroRegions z{};
     z.p[0] = res.counters;
     z.n[0] = kCounterWords;
-    const PassPlan pp = pass_plan(plan, views, n_views);
+    const MarchPlan &mp = plan.march;
+    const uint32_t subs = mp.n ? mp.subs : kRefineSubs;
+    const MarchBuffers mb{res.view_table, res.cont_buf, (uint32_t *)res.cont_counts, res.refine_buf,
+                          (uint32_t *)res.refine_counts, res.counters};
     z.p[1] = (uint32_t *)res.cont_counts;
-    z.n[1] = pp.n ? (pp.n + 1u) * n_views * kContSubs * kHeadStride : 3u * n_views;
+    z.n[1] = mp.n ? (mp.n + 1u) * n_views * subs * kHeadStride : 3u * n_views;
     z.p[2] = park ? (uint32_t *)res.refine_counts : nullptr;
-    z.n[2] = park ? n_views * kRefineSubs * kHeadStride : 0u;
-    z.p[3] = (uint32_t *)res.vox_counts;
-    z.n[3] = n_views * kHeadStride;
-    const uint32_t zmax = std::max(std::max(z.n[0], z.n[1]), std::max(z.n[2], z.n[3]));
-    hipLaunchKernelGGL(zero_regions, dim3((zmax + 255u) / 256u, 4), dim3(256), 0, ctx->stream, z);
+    z.n[2] = park ? n_views * subs * kHeadStride : 0u;
+    const uint32_t zmax = std::max(z.n[0], std::max(z.n[1], z.n[2]));
+    hipLaunchKernelGGL(zero_regions, dim3((zmax + 255u) / 256u, 3), dim3(256), 0, ctx->stream, z);
     LYAP_HIP(ctx, hipGetLastError());
     int rc = LYAP_OK;
-    uint64_t cap_total = 0, list_total = 0, lanes0 = 0;
-    bool has_rays = false;
+    uint64_t cap_total = 0, lanes0 = 0;
     for (unsigned i = 0; i < n_views; ++i) {
         cap_total += views[i].cont_cap;
-        list_total += views[i].vlist_cap;
-        if (views[i].kind == kItemView) {
-            has_rays = true;
-            lanes0 += (uint64_t)views[i].n_tiles * plan.tile_rays * plan.lanes_per_ray;
-        } else {
-            lanes0 += (uint64_t)views[i].n_tiles * 64u;
-        }
+        lanes0 += (uint64_t)views[i].n_tiles * plan.tile_rays * plan.lanes_per_ray;
     }
     ContEntry *bufA = (ContEntry *)res.cont_buf;
     ContEntry *bufB = bufA + cap_total;
@@ -2395,8 +1536,7 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
     /* level l reads the rays level l-1 handed over (buffers alternate) */
     ContEntry *out_buf[4] = {bufA, bufB, bufA, nullptr};
     const ContEntry *in_buf[4] = {nullptr, bufA, bufB, bufA};
-    /* volume blocks finish at level 0; later levels carry rays only */
-    uint32_t levels = (plan.direct || !has_rays) ? 1u : 4u;
+    uint32_t levels = plan.direct ? 1u : 4u;
     uint32_t first_level = 0;
     if (walks(plan, views, n_views)) {
         uint64_t rays = 0;
@@ -2407,9 +1547,9 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
         if (rc) return rc;
         return timing_mark(ctx);
     }
-    if (pp.n > 0) {
+    if (mp.n > 0) {
         /* the passes march every ray to its end: no level launch follows */
-        rc = enqueue_passes(ctx, res, views, n_views, pp, W, precision);
+        rc = launch_march(ctx, views, n_views, mp, mb, W, precision);
         if (rc) return rc;
         first_level = levels;
     }
@@ -2433,8 +1573,6 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
         a.out_counts = level < 3 ? counts + level * n_views : nullptr;
         a.refine_out = park ? (RefineRec *)res.refine_buf : nullptr;
         a.refine_counts = park ? (uint32_t *)res.refine_counts : nullptr;
-        a.vox_list = (uint32_t *)res.vox_list;
-        a.vox_counts = (uint32_t *)res.vox_counts;
         uint32_t blocks = plan.blocks;
         if (level == 0 && blocks > needed0) blocks = (uint32_t)needed0;
         if (blocks == 0) blocks = 1;
@@ -2459,26 +1597,13 @@ static int enqueue_views(lyap_ctx *ctx, RenderResources &res, const ViewDesc *vi
         LYAP_HIP(ctx, hipGetLastError());
         rc = timing_mark(ctx);
         if (rc) return rc;
-        if (level == 0 && list_total > 0) {
-            /* FP64 re-evaluation of the voxels the blocks listed */
-            VoxelFp64Args va{};
-            va.n_items = n_views;
-            va.list = (const uint32_t *)res.vox_list;
-            va.counts = (const uint32_t *)res.vox_counts;
-            const uint32_t vb = (uint32_t)std::min<uint64_t>(cus * 8u, (list_total + 255u) / 256u);
-            if (W == 16)
-                hipLaunchKernelGGL(voxel_fp64<16>, dim3(vb), dim3(256), 0, ctx->stream,
-                                   (const ViewDesc *)res.view_table, va);
-            else
-                hipLaunchKernelGGL(voxel_fp64<32>, dim3(vb), dim3(256), 0, ctx->stream,
-                                   (const ViewDesc *)res.view_table, va);
-            LYAP_HIP(ctx, hipGetLastError());
-        }
     }
-    if (park && has_rays) {
+    if (park) {
         rc = timing_mark(ctx);
         if (rc) return rc;
-        rc = launch_refine(ctx, res, n_views, W, precision, margin);
+        uint64_t rays = 0;
+        for (unsigned i = 0; i < n_views; ++i) rays += views[i].n_rays;
+        rc = launch_refine(ctx, n_views, subs, rays, mb, W, precision, margin);
         if (rc) return rc;
         rc = timing_mark(ctx);
         if (rc) return rc;
@@ -2566,10 +1691,8 @@ static int build_batch(lyap_ctx *ctx, const LyapView *in, unsigned n, const Lyap
     return LYAP_OK;
 }
 
-/* Appends the validated volume blocks to a launch's items (after its views)
- * and widens the coefficient window if a block's sequence needs it. */
-static int append_blocks(lyap_ctx *ctx, const LyapVolumeBlock *in, unsigned n,
-                         const LyapVolumeMode &vmode, std::vector<ViewDesc> &items, uint32_t &W)
+/* Validates the volume blocks of a batch. */
+static int check_blocks(lyap_ctx *ctx, const LyapVolumeBlock *in, unsigned n)
 {
     for (unsigned i = 0; i < n; ++i) {
         const LyapVolumeBlock &b = in[i];
@@ -2583,10 +1706,28 @@ static int append_blocks(lyap_ctx *ctx, const LyapVolumeBlock *in, unsigned n,
         if (!make_eval_desc(&e, b.prm, b.seq))
             return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "volume block %u: sequence must hold 1..%d letter "
                         "indices 0..3 before the -1", i, LYAP_MAX_SEQ);
-        ViewDesc v;
-        fill_block(v, e, b.prm, b.lo, b.hi, b.n, b.z_begin, z1, b.out, vmode);
-        items.push_back(v);
-        if (e.L > 16) W = 32;
+    }
+    return LYAP_OK;
+}
+
+/* The blocks of a batch through the volume kernels, on the context's stream
+ * after the views: a kernel specialised on the period, in bricks that settle
+ * together, at eight waves per SIMD. As tiles of the views' persistent launch
+ * (three waves per SIMD, rows, the window's blocks) 64 views with eight 128^3
+ * blocks took as long as views and blocks apart. totals (device memory, one
+ * word per block, or null): voxels re-evaluated. */
+int launch_blocks(lyap_ctx *ctx, const LyapVolumeBlock *blocks, unsigned n, const LyapVolumeMode &vmode,
+                  uint32_t *totals)
+{
+    for (unsigned i = 0; i < n; ++i) {
+        const LyapVolumeBlock &b = blocks[i];
+        EvalDesc e;
+        if (!make_eval_desc(&e, b.prm, b.seq))
+            return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "volume block %u: bad sequence", i);
+        const uint32_t z1 = b.z_end ? b.z_end : b.n[2];
+        int rc = launch_volume_slab(ctx, b.out, e, b.lo, b.hi, b.n[0], b.n[1], b.n[2], b.z_begin, z1,
+                                    nullptr, 0, vmode, totals ? totals + i : nullptr);
+        if (rc) return rc;
     }
     return LYAP_OK;
 }
@@ -2595,12 +1736,11 @@ static int render_views(lyap_ctx *ctx, std::vector<ViewDesc> &views, uint32_t W,
                         const LyapRenderMode &mode, const LyapTuning &tune)
 {
     uint64_t rays = 0;
-    for (auto &v : views)
-        if (v.kind == kItemView) rays += v.n_rays;
+    for (auto &v : views) rays += v.n_rays;
     const bool margin = mode.fp64_margin > 0.0f && mode.refine == LYAP_REFINE_BISECT;
     LyapTuning t = tune;
     if (!t.lanes_per_ray && mode.lanes_per_ray) t.lanes_per_ray = mode.lanes_per_ray;
-    const LaunchPlan plan = plan_launch(ctx, rays, t, W, mode.precision, margin,
+    LaunchPlan plan = plan_launch(ctx, rays, t, W, mode.precision, margin,
                                         mode.schedule == LYAP_SCHEDULE_DIRECT,
                                         mode.schedule == LYAP_SCHEDULE_LEVELS);
     RenderResources &res = ctx_resources(ctx);
@@ -2612,6 +1752,7 @@ static int render_views(lyap_ctx *ctx, std::vector<ViewDesc> &views, uint32_t W,
     /* lyap_last_evals reads this frame's counters (a capture, which
      * enqueues without running, leaves the previous call's in place) */
     ctx->last_counters = res.counters;
+    ctx->last_voxels = 0;
     LYAP_HIP(ctx, hipEventRecord(res.staged[res.stage], ctx->stream));
     return LYAP_OK;
 }
@@ -2662,28 +1803,14 @@ void render_slot_destroy(lyap_ctx *ctx, RenderSlot *slot)
 
 const uint32_t *render_slot_counters(const RenderSlot *slot) { return slot->res.counters; }
 
-const uint32_t *render_slot_vox_counts(const RenderSlot *slot)
-{
-    return static_cast<const uint32_t *>(slot->res.vox_counts);
-}
-
-static_assert(kItemCountStride == kHeadStride, "per-item counter spacing");
-
 /* Renders rays [ray_begin[i], ray_begin[i] + ray_count[i]) of views[i] for
- * every i, in that order of priority, then the volume blocks (items n ..
- * n + nb - 1 of the launch), with the slot's own resources. The blocks must
- * use the views' precision (or there are no views). The caller guarantees
- * the slot's previous launch has finished, so nothing here waits on the
- * device. ray_begin is a multiple of 64 (whole 8x8 blocks). */
+ * every i, in that order of priority, with the slot's own resources. The
+ * caller guarantees the slot's previous launch has finished, so nothing here
+ * waits on the device. ray_begin is a multiple of 64 (whole 8x8 blocks). */
 int render_slot_launch(lyap_ctx *ctx, RenderSlot *slot, const LyapView *in,
                        const uint32_t *ray_begin, const uint32_t *ray_count, unsigned n,
-                       const LyapVolumeBlock *blocks, unsigned nb, const LyapVolumeMode &vmode,
-                       const LyapRenderMode &mode_in, const LyapTuning &tune)
+                       const LyapRenderMode &mode, const LyapTuning &tune)
 {
-    LyapRenderMode mode = mode_in;
-    if (n == 0) mode.precision = vmode.precision;
-    if (nb && mode.precision != vmode.precision)
-        return fail(ctx, LYAP_ERR_UNSUPPORTED, "volume blocks need the views' precision in one launch");
     std::vector<ViewDesc> views(n);
     uint32_t maxL = 1;
     uint64_t rays = 0;
@@ -2695,22 +1822,20 @@ int render_slot_launch(lyap_ctx *ctx, RenderSlot *slot, const LyapView *in,
         rays += ray_count[i];
         if ((uint32_t)views[i].e.L > maxL) maxL = (uint32_t)views[i].e.L;
     }
-    uint32_t W = maxL <= 16 ? 16u : 32u;
-    int rc = append_blocks(ctx, blocks, nb, vmode, views, W);
-    if (rc) return rc;
+    const uint32_t W = maxL <= 16 ? 16u : 32u;
     const bool margin = mode.fp64_margin > 0.0f && mode.refine == LYAP_REFINE_BISECT;
     LyapTuning t = tune;
     if (!t.lanes_per_ray && mode.lanes_per_ray) t.lanes_per_ray = mode.lanes_per_ray;
-    const LaunchPlan plan = plan_launch(ctx, rays, t, W, mode.precision, margin,
+    LaunchPlan plan = plan_launch(ctx, rays, t, W, mode.precision, margin,
                                         mode.schedule == LYAP_SCHEDULE_DIRECT,
                                         mode.schedule == LYAP_SCHEDULE_LEVELS);
     uint32_t total_tiles = 0;
-    const unsigned items = (unsigned)views.size();
-    rc = prepare_views(ctx, slot->res, views.data(), items, plan, W, false, &total_tiles);
+    int rc = prepare_views(ctx, slot->res, views.data(), n, plan, W, false, &total_tiles);
     if (rc) return rc;
-    rc = enqueue_views(ctx, slot->res, views.data(), items, total_tiles, plan, W, mode.precision);
+    rc = enqueue_views(ctx, slot->res, views.data(), n, total_tiles, plan, W, mode.precision);
     if (rc) return rc;
     ctx->last_counters = slot->res.counters;
+    ctx->last_voxels = 0;
     return LYAP_OK;
 }
 
@@ -2833,42 +1958,6 @@ static int check_volume_mode(lyap_ctx *ctx, const LyapVolumeMode *in, LyapVolume
     return LYAP_OK;
 }
 
-/* The items of a mixed launch (views sorted, then blocks) and the render
- * mode the launch runs in: the views' precision, or the blocks' when there
- * are no views. `fused` is false when the blocks need another precision than
- * the views; they are then left out of `items`. */
-static int build_mixed(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
-                       const LyapVolumeBlock *blocks, unsigned n_blocks, const LyapRenderMode &mode,
-                       const LyapVolumeMode &vmode, std::vector<ViewDesc> &items, uint32_t &W,
-                       LyapRenderMode &launch_mode, bool &fused)
-{
-    int rc = build_batch(ctx, views, n_views, mode, items, W);
-    if (rc) return rc;
-    launch_mode = mode;
-    fused = n_blocks == 0 || n_views == 0 || vmode.precision == mode.precision;
-    if (n_views == 0) launch_mode.precision = vmode.precision;
-    if (fused) return append_blocks(ctx, blocks, n_blocks, vmode, items, W);
-    return LYAP_OK;
-}
-
-/* The blocks of a batch whose precision differs from the views': through
- * the volume kernels, on the context's stream after the views. */
-static int run_blocks_apart(lyap_ctx *ctx, const LyapVolumeBlock *blocks, unsigned n,
-                            const LyapVolumeMode &vmode)
-{
-    for (unsigned i = 0; i < n; ++i) {
-        const LyapVolumeBlock &b = blocks[i];
-        EvalDesc e;
-        if (!make_eval_desc(&e, b.prm, b.seq))
-            return fail(ctx, LYAP_ERR_BAD_SEQUENCE, "volume block %u: bad sequence", i);
-        const uint32_t z1 = b.z_end ? b.z_end : b.n[2];
-        int rc = launch_volume_slab(ctx, b.out, e, b.lo, b.hi, b.n[0], b.n[1], b.n[2], b.z_begin, z1,
-                                    nullptr, 0, vmode);
-        if (rc) return rc;
-    }
-    return LYAP_OK;
-}
-
 } /* namespace lyap */
 
 extern "C" int lyap_run_batch(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
@@ -2886,16 +1975,32 @@ extern "C" int lyap_run_batch(lyap_ctx *ctx, const LyapView *views, unsigned n_v
     LyapVolumeMode vmode;
     rc = check_volume_mode(ctx, vol_mode_in, vmode);
     if (rc) return rc;
-    std::vector<ViewDesc> items;
+    std::vector<ViewDesc> vd;
     uint32_t W;
-    LyapRenderMode lmode;
-    bool fused;
-    rc = build_mixed(ctx, views, n_views, blocks, n_blocks, mode, vmode, items, W, lmode, fused);
+    rc = build_batch(ctx, views, n_views, mode, vd, W);
     if (rc) return rc;
-    rc = render_views(ctx, items, W, lmode, merged_tuning(ctx, tuning));
+    rc = check_blocks(ctx, blocks, n_blocks);
     if (rc) return rc;
-    if (!fused) return run_blocks_apart(ctx, blocks, n_blocks, vmode);
-    return LYAP_OK;
+    /* the largest block's re-evaluation list exists before anything runs */
+    uint64_t voxels = 0, largest = 0;
+    for (unsigned i = 0; i < n_blocks; ++i) {
+        const LyapVolumeBlock &b = blocks[i];
+        const uint64_t nb = (uint64_t)b.n[0] * b.n[1] * ((b.z_end ? b.z_end : b.n[2]) - b.z_begin);
+        voxels += nb;
+        largest = std::max(largest, nb);
+    }
+    if (has_rule(vmode) && largest > 0 && largest <= 0xFFFFFFFFull) {
+        rc = ensure_reeval_list(ctx, largest);
+        if (rc) return rc;
+    }
+    if (n_views) {
+        rc = render_views(ctx, vd, W, mode, merged_tuning(ctx, tuning));
+        if (rc) return rc;
+    } else {
+        ctx->last_counters = nullptr;
+    }
+    ctx->last_voxels = voxels;
+    return launch_blocks(ctx, blocks, n_blocks, vmode, nullptr);
 }
 
 namespace lyap {
@@ -2921,9 +2026,9 @@ static int time_items(lyap_ctx *ctx, const std::vector<ViewDesc> &items, uint32_
 }
 
 /* The staged search of lyap_autotune_batch: launch shape, then the level
- * budgets one level at a time, then the voxel tile. */
+ * budgets one level at a time. */
 static int autotune_items(lyap_ctx *ctx, const std::vector<ViewDesc> &items, uint32_t W,
-                          const LyapRenderMode &mode, bool has_rays, bool has_blocks, LyapTuning &best_t)
+                          const LyapRenderMode &mode, LyapTuning &best_t)
 {
     hipEvent_t e0, e1;
     LYAP_HIP(ctx, hipEventCreate(&e0));
@@ -2940,36 +2045,26 @@ static int autotune_items(lyap_ctx *ctx, const std::vector<ViewDesc> &items, uin
     };
     best_t = LyapTuning{};
     trial(best_t);                                  /* the built-in shape */
-    if (has_rays) {
-        /* samples per ray and round K x S from 1 (one lane per ray) to 16,
-         * tiles of one or two generations of a wave's groups */
-        const uint32_t shapes[][2] = {{1, 1}, {2, 1}, {4, 1}, {8, 1}, {16, 1}, {1, 2}, {2, 2}, {4, 2}, {1, 4}};
-        const LyapTuning base = best_t;
-        for (const auto &sh : shapes) {
-            for (uint32_t g : {1u, 2u}) {
-                LyapTuning t = base;
-                t.lanes_per_ray = sh[0];
-                t.slots = sh[1];
-                t.tile_rays = g * (64u / sh[0]);
-                trial(t);
-            }
-        }
-        /* march-sample budgets of levels 0, 1 and 2, one level at a time */
-        const uint32_t cand[3][4] = {{16, 24, 32, 64}, {32, 48, 64, 96}, {96, 128, 192, 256}};
-        for (int lv = 0; lv < 3 && rc == LYAP_OK; ++lv) {
-            const LyapTuning base2 = best_t;
-            for (uint32_t b : cand[lv]) {
-                LyapTuning t = base2;
-                t.level_budget[lv] = b;
-                trial(t);
-            }
+    /* samples per ray and round K x S from 1 (one lane per ray) to 16,
+     * tiles of one or two generations of a wave's groups */
+    const uint32_t shapes[][2] = {{1, 1}, {2, 1}, {4, 1}, {8, 1}, {16, 1}, {1, 2}, {2, 2}, {4, 2}, {1, 4}};
+    const LyapTuning base = best_t;
+    for (const auto &sh : shapes) {
+        for (uint32_t g : {1u, 2u}) {
+            LyapTuning t = base;
+            t.lanes_per_ray = sh[0];
+            t.slots = sh[1];
+            t.tile_rays = g * (64u / sh[0]);
+            trial(t);
         }
     }
-    if (has_blocks) {
-        const LyapTuning base = best_t;
-        for (uint32_t vt : {64u, 128u, 512u, 1024u}) {
-            LyapTuning t = base;
-            t.voxel_tile = vt;
+    /* march-sample budgets of levels 0, 1 and 2, one level at a time */
+    const uint32_t cand[3][4] = {{16, 24, 32, 64}, {32, 48, 64, 96}, {96, 128, 192, 256}};
+    for (int lv = 0; lv < 3 && rc == LYAP_OK; ++lv) {
+        const LyapTuning base2 = best_t;
+        for (uint32_t b : cand[lv]) {
+            LyapTuning t = base2;
+            t.level_budget[lv] = b;
             trial(t);
         }
     }
@@ -2996,12 +2091,13 @@ extern "C" int lyap_autotune_batch(lyap_ctx *ctx, const LyapView *views, unsigne
     if (rc) return rc;
     std::vector<ViewDesc> items;
     uint32_t W;
-    LyapRenderMode lmode;
-    bool fused;
-    rc = build_mixed(ctx, views, n_views, blocks, n_blocks, mode, vmode, items, W, lmode, fused);
+    rc = build_batch(ctx, views, n_views, mode, items, W);
+    if (rc) return rc;
+    rc = check_blocks(ctx, blocks, n_blocks);
     if (rc) return rc;
     LyapTuning t{};
-    rc = autotune_items(ctx, items, W, lmode, n_views > 0, fused && n_blocks > 0, t);
+    /* the blocks run in the volume kernels, which have no shape to choose */
+    if (n_views) rc = autotune_items(ctx, items, W, mode, t);
     if (rc) return rc;
     ctx->tuned = t;
     if (best) *best = t;
@@ -3047,7 +2143,7 @@ extern "C" int lyap_frame_capture(lyap_ctx *ctx, const LyapView *views, unsigned
     uint64_t rays = 0;
     for (auto &v : vd) rays += v.n_rays;
     const bool margin = mode.fp64_margin > 0.0f && mode.refine == LYAP_REFINE_BISECT;
-    const LaunchPlan plan = plan_launch(ctx, rays, merged_tuning(ctx, tuning), W, mode.precision, margin,
+    LaunchPlan plan = plan_launch(ctx, rays, merged_tuning(ctx, tuning), W, mode.precision, margin,
                                         mode.schedule == LYAP_SCHEDULE_DIRECT,
                                         mode.schedule == LYAP_SCHEDULE_LEVELS);
     lyap_frame *f = new lyap_frame();
@@ -3091,6 +2187,7 @@ extern "C" int lyap_frame_replay(lyap_ctx *ctx, lyap_frame *f)
     if (!ctx || !f || f->ctx != ctx || !f->exec) return LYAP_ERR_INVALID_ARGUMENT;
     LYAP_HIP(ctx, hipGraphLaunch(f->exec, ctx->stream));
     ctx->last_counters = f->res.counters;
+    ctx->last_voxels = 0;
     return LYAP_OK;
 }
 

@@ -36,24 +36,10 @@ struct ViewDesc {
     uint32_t cont_base;        /* this view's region of the continuation buffers */
     uint32_t cont_cap;
     uint32_t refine_base;      /* this view's region of the refinement records */
-    uint32_t refine_cap;       /* records per sub-region (kRefineSubs of them) */
+    uint32_t refine_cap;       /* records per sub-list */
     uint32_t ray_base;         /* first ray of this view in a grid of one lane per ray */
-    /* Items of a launch are views or volume blocks (kItemVolume). A volume
-     * block is z slices [vz0, vz0 + n_rays / (vnx * vny)) of an vnx * vny * vnz
-     * grid over [vlo, vlo + vspan), lambda written to vol_out (slice vz0) in
-     * the x-fastest layout of kernel.cu:525; voxels the FP32 pass is unsure of
-     * go to the block's region of the FP64 list. */
-    uint32_t kind;
-    uint32_t tile_len;         /* rays or voxels per level-0 work-queue tile */
-    float *vol_out;
-    uint32_t vnx, vny, vnz, vz0;
-    float vlo[3], vspan[3];
-    float vmargin, vtau, vband;
-    uint32_t vlist_base, vlist_cap;
+    uint32_t tile_len;         /* rays per level-0 work-queue tile */
 };
-
-constexpr uint32_t kItemView = 0;
-constexpr uint32_t kItemVolume = 1;
 
 /* Words between counters that different waves update: one 128-byte line. */
 constexpr uint32_t kHeadStride = 32;
@@ -68,17 +54,12 @@ struct alignas(16) RefineRec {
 };
 static_assert(sizeof(RefineRec) == 48, "refinement record size");
 
-/* Refinement records of a view are kept in kRefineSubs sub-regions, one per
- * block index modulo kRefineSubs, each with its own counter on a 128-byte
- * line: waves of one XCD share a counter, and device-scope atomics on a line
- * that waves of several XCDs update are slow. */
+/* The refinement records of a view are kept in sub-lists with a counter each
+ * on a 128-byte line, taken by block index: waves of one XCD share a counter
+ * (device-scope atomics on a line that waves of several XCDs update are
+ * slow). The persistent levels use kRefineSubs, the march passes
+ * MarchPlan::subs for these and for the rays they list. */
 constexpr uint32_t kRefineSubs = 8;
-
-/* The march passes list their rays the same way: a view's continuation
- * region is kContSubs sub-lists of cont_cap / kContSubs records, one counter
- * per sub-list on its own 128-byte line, taken by block index modulo
- * kContSubs. */
-constexpr uint32_t kContSubs = 8;
 
 struct F3 { float x, y, z; };
 __device__ __forceinline__ F3 f3(const LyapVec &v) { return {v.x, v.y, v.z}; }
@@ -310,6 +291,31 @@ __device__ __forceinline__ void count_evals(unsigned long long *counter, unsigne
     for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off);
     if (__lane_id() == 0 && n) atomicAdd(counter + wid % kEvalSlots * kEvalStride, n);
 }
+
+/* march.hip */
+constexpr uint32_t kMaxPasses = 16;
+constexpr size_t kPassRecBytes = 48;
+struct MarchPlan {
+    uint32_t n = 0;                   /* passes after the first; 0: the persistent levels */
+    uint32_t subs = 0;                /* sub-lists per view */
+    uint32_t K[kMaxPasses] = {};      /* lanes per ray of each pass, at least */
+    uint32_t R[kMaxPasses] = {};      /* rounds of each pass (0: until the rays end) */
+};
+/* `rays`: of all views. */
+MarchPlan march_plan(unsigned n_views, uint64_t rays);
+/* Device memory of a launch's marching and parked rays. */
+struct MarchBuffers {
+    const void *view_table;
+    void *cont;                       /* 2 x the views' cont_cap records */
+    uint32_t *cont_counts;
+    void *refine;
+    uint32_t *refine_counts;
+    uint32_t *counters;               /* evaluation counts */
+};
+int launch_march(lyap_ctx *ctx, const ViewDesc *views, unsigned n_views, const MarchPlan &mp,
+                 const MarchBuffers &b, uint32_t W, int precision);
+int launch_refine(lyap_ctx *ctx, unsigned n_views, uint32_t subs, uint64_t rays, const MarchBuffers &b,
+                  uint32_t W, int precision, bool margin);
 
 /* walk.hip */
 int launch_walk(lyap_ctx *ctx, const void *view_table, unsigned n_views, uint64_t rays, uint32_t *counters,

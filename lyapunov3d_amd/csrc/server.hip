@@ -35,11 +35,13 @@ struct HipSlot {
     int kind = SLOT_MIXED;
     RenderSlot *rs = nullptr;
     hipEvent_t start = nullptr, end = nullptr;
-    /* pinned: the launch's lambda evaluations (rays' samples, one per voxel) */
-    uint64_t *host_evals = nullptr;   /* kEvalSlots counts (a volume slot: word 0) */
-    /* pinned: FP64 re-evaluations of each slab, kItemCountStride words apart */
-    uint32_t *host_reeval = nullptr;
+    /* pinned: the lambda evaluations of the launch's views */
+    uint64_t *host_evals = nullptr;   /* kEvalSlots counts */
+    /* FP64 re-evaluations of each slab: on the device and pinned */
+    uint32_t *reeval = nullptr, *host_reeval = nullptr;
     unsigned nblocks = 0;
+    bool has_views = false;
+    uint64_t voxels = 0;
 };
 
 class HipBackend final : public ServeBackend {
@@ -58,7 +60,7 @@ public:
             sl.kind = kinds[i];
             int rc = lyap_create(&sl.ctx, owner_->device, 0);
             if (rc) return fail(owner_, rc, "server slot context: %s", lyap_strerror(rc));
-            const size_t reeval_bytes = kMaxSlabs * kItemCountStride * sizeof(uint32_t);
+            const size_t reeval_bytes = kMaxSlabs * sizeof(uint32_t);
             if (hipEventCreate(&sl.start) != hipSuccess || hipEventCreate(&sl.end) != hipSuccess ||
                 hipHostMalloc((void **)&sl.host_evals, kEvalBytes, hipHostMallocDefault) !=
                     hipSuccess ||
@@ -66,17 +68,18 @@ public:
                 return fail(owner_, LYAP_ERR_DEVICE, "server slot set-up failed");
             std::memset(sl.host_evals, 0, kEvalBytes);
             std::memset(sl.host_reeval, 0, reeval_bytes);
-            if (sl.kind != SLOT_VOLUME) {
-                sl.rs = render_slot_create();
-            } else if (cfg_.vol_mode.precision == LYAP_PREC_PRODUCT &&
-                       (cfg_.vol_mode.fp64_margin > 0.0f || cfg_.vol_mode.converge_tau > 0.0f)) {
+            if (sl.kind != SLOT_VOLUME) sl.rs = render_slot_create();
+            if (sl.kind != SLOT_RENDER && has_rule(cfg_.vol_mode)) {
                 /* re-evaluation list for the largest slab (256 x 256 x 256) up
                  * front, so a slab never reallocates while others run */
                 rc = ensure_reeval_list(sl.ctx, 256u * 256u * 256u);
+                void *p = nullptr;
+                if (rc == LYAP_OK) rc = ctx_alloc(sl.ctx, &p, reeval_bytes);
                 if (rc) {
                     owner_->last_error = sl.ctx->last_error;
                     return rc;
                 }
+                sl.reeval = (uint32_t *)p;
             }
         }
         return LYAP_OK;
@@ -124,9 +127,9 @@ public:
         if (q != hipSuccess) return fail(owner_, LYAP_ERR_DEVICE, "server launch: %s", hipGetErrorString(q));
         float ms = 0.0f;
         res->ms = hipEventElapsedTime(&ms, sl.start, sl.end) == hipSuccess ? (double)ms : -1.0;
-        res->evals = sl.kind == SLOT_VOLUME ? sl.host_evals[0] : sum_evals(sl.host_evals);
+        res->evals = sl.voxels + (sl.has_views ? sum_evals(sl.host_evals) : 0u);
         for (unsigned b = 0; b < sl.nblocks && b < kMaxSlabs; ++b)
-            res->reeval[b] = sl.host_reeval[b * kItemCountStride];
+            res->reeval[b] = sl.host_reeval[b];
         return LYAP_OK;
     }
 
@@ -144,35 +147,21 @@ private:
     int launch_on(HipSlot &sl, const SlotLaunch &l)
     {
         sl.nblocks = (unsigned)l.blocks.size();
+        sl.has_views = !l.views.empty();
+        sl.voxels = l.voxels;
         LYAP_HIP(sl.ctx, hipEventRecord(sl.start, sl.ctx->stream));
-        if (sl.kind == SLOT_VOLUME) {
-            /* the volume kernels, slab by slab; each slab's re-evaluation
-             * count (the counter restarts per slab) */
-            for (size_t b = 0; b < l.blocks.size(); ++b) {
-                const LyapVolumeBlock &k = l.blocks[b];
-                EvalDesc e;
-                if (!make_eval_desc(&e, k.prm, k.seq))
-                    return fail(sl.ctx, LYAP_ERR_BAD_SEQUENCE, "bad sequence");
-                int rc = launch_volume_slab(sl.ctx, k.out, e, k.lo, k.hi, k.n[0], k.n[1], k.n[2], k.z_begin,
-                                            k.z_end, nullptr, 0, cfg_.vol_mode);
-                if (rc) return rc;
-                sl.host_reeval[b * kItemCountStride] = 0;
-                if (sl.ctx->has_reevaluated)
-                    LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval + b * kItemCountStride, sl.ctx->counters + kReevalWords, 4,
-                                                    hipMemcpyDeviceToHost, sl.ctx->stream));
-            }
-            *sl.host_evals = l.voxels;
-        } else {
+        if (sl.has_views) {
             int rc = render_slot_launch(sl.ctx, sl.rs, l.views.data(), l.begin.data(), l.count.data(),
-                                        (unsigned)l.views.size(), l.blocks.data(), (unsigned)l.blocks.size(),
-                                        cfg_.vol_mode, cfg_.mode, owner_->tuned);
+                                        (unsigned)l.views.size(), cfg_.mode, owner_->tuned);
             if (rc) return rc;
             LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_evals, render_slot_counters(sl.rs), kEvalBytes,
                                             hipMemcpyDeviceToHost, sl.ctx->stream));
-            if (!l.blocks.empty())
-                LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval,
-                                                render_slot_vox_counts(sl.rs) + l.views.size() * kItemCountStride,
-                                                l.blocks.size() * kItemCountStride * sizeof(uint32_t),
+        }
+        if (sl.nblocks) {
+            int rc = launch_blocks(sl.ctx, l.blocks.data(), sl.nblocks, cfg_.vol_mode, sl.reeval);
+            if (rc) return rc;
+            if (has_rule(cfg_.vol_mode))
+                LYAP_HIP(sl.ctx, hipMemcpyAsync(sl.host_reeval, sl.reeval, sl.nblocks * sizeof(uint32_t),
                                                 hipMemcpyDeviceToHost, sl.ctx->stream));
         }
         LYAP_HIP(sl.ctx, hipEventRecord(sl.end, sl.ctx->stream));
