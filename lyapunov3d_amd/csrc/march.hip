@@ -358,9 +358,13 @@ __global__ __launch_bounds__(64) void march_start(const ViewDesc *__restrict__ v
     count_evals(a.eval_counter, state == R_MISS ? evals : 0u, blockIdx.x);
 }
 
-/* `rounds` rounds (0: until the march ends) for every listed ray. */
+/* `rounds` rounds (0: until the march ends) for every listed ray. Vector
+ * instructions bound it, and six waves per SIMD run them best: five (90
+ * registers) take 857 us for a frame of 1024x1024 and 326 for 512x512, six 830
+ * and 325, eight, with registers spilled, 831 and 337. */
 template <int W, int PREC>
-__global__ __launch_bounds__(256) void march_pass(const ViewDesc *__restrict__ views, PassArgs a)
+__global__ __launch_bounds__(256, W == 16 && PREC == LYAP_PREC_PRODUCT ? 6 : 1)
+void march_pass(const ViewDesc *__restrict__ views, PassArgs a)
 {
     __shared__ Shares shares[4];
     Shares &sh = shares[threadIdx.x >> 6];
@@ -449,12 +453,15 @@ __device__ __forceinline__ float refine_eval(const ViewDesc &v, F3 sp, float thr
  * the first sample chooses, the trip resolves two levels. The normal then
  * takes three trips, the minus samples on the first lane and the plus samples
  * on the second. The arithmetic is the march kernel's, step for step, so the
- * bytes are those of refining in place. Two lanes halve a small launch's
+ * bytes are those of refining in place. Vector instructions bound it (a record
+ * is read once per 14 samples), so registers are held to eight waves per SIMD:
+ * 64 frames of 512x512 44.0 ms against 46.6 with seven. Two lanes halve a small launch's
  * chain of evaluations; one lane evaluates nothing it does not need (14
  * samples a ray instead of about 17), which a launch that fills the chip many
  * times over is bound by. */
 template <int W, int PREC, bool MARGIN, int G>
-__global__ __launch_bounds__(256) void refine_rays(const ViewDesc *__restrict__ views, RefineArgs a)
+__global__ __launch_bounds__(256, W == 16 && PREC == LYAP_PREC_PRODUCT && !MARGIN ? 8 : 1)
+void refine_rays(const ViewDesc *__restrict__ views, RefineArgs a)
 {
     constexpr uint32_t per = 64u / G;
     const uint32_t lane = __lane_id();
@@ -580,11 +587,15 @@ __global__ __launch_bounds__(256) void refine_rays(const ViewDesc *__restrict__ 
  * ray's end costs what a needed one does: one lane per ray for as long as
  * enough rays march, in passes short enough that the lanes of ended rays do
  * not idle long, and one refining lane. Both sides, few / many, in us per
- * frame: 256x256 263 / 316, 512x512 320 / 370, 1024x1024 847 / 853, 1448x1448
- * 1585 / 1495, 2048x2048 3050 / 2705; 64 frames of 512x512 51400 / 44400. The
+ * frame: 256x256 265 / 335, 512x512 320 / 371, 1024x1024 796 / 864, 1448x1448
+ * 1499 / 1464, 2048x2048 2900 / 2584; 64 frames of 512x512 48700 / 38600. The
  * march kernel in levels takes 355, 509 and 1765 us for the first three and
  * 51900 for the 64. */
-constexpr uint64_t kManyRays = 1200000;
+constexpr uint64_t kManyRays = 1800000;
+/* Blocks: a pass of many rays gets kManyTurns grids' worth, and the refinement
+ * several per slot, so that a slot whose blocks had cheap rays takes another
+ * one: 64 frames of 512x512 take 41.4 ms with one grid each and 37.3 so. */
+constexpr uint32_t kManyTurns = 4, kFewRefine = 16, kManyRefine = 64;
 const char *const kFewPasses = "2x4,4x4,8x4,16x4,32x4,64x4,64x0";
 const char *const kManyPasses = "1x4,1x4,1x8,1x8,1x16,1x16,2x16,2x16,4x16,8x16,16x8,64x0";
 
@@ -639,14 +650,16 @@ static uint32_t pass_blocks_per_cu()
 int launch_march(lyap_ctx *ctx, const ViewDesc *views, unsigned n_views, const MarchPlan &mp,
                  const MarchBuffers &b, uint32_t W, int precision)
 {
-    uint64_t cap_total = 0, rays = 0;
+    uint64_t cap_total = 0, rays = 0, all = 0;
     for (unsigned i = 0; i < n_views; ++i) {
         cap_total += views[i].cont_cap;
+        all += views[i].n_rays;
         rays += (views[i].n_rays + 255u) / 256u * 256u;
     }
     PassRec *buf[2] = {(PassRec *)b.cont, (PassRec *)b.cont + cap_total};
     const uint32_t pass_words = n_views * mp.subs * kHeadStride;
     const uint32_t cus = ctx->num_cus > 0 ? (uint32_t)ctx->num_cus : 256u;
+    const uint32_t turns = all >= kManyRays ? kManyTurns : 1u;
     PassArgs a{};
     a.n_views = n_views;
     a.subs = mp.subs;
@@ -687,7 +700,7 @@ int launch_march(lyap_ctx *ctx, const ViewDesc *views, unsigned n_views, const M
     do {                                                                                               \
         const uint32_t blocks = cus * pass_blocks_per_cu<WW, PP>();                                    \
         a.lanes = blocks * 256u;                                                                       \
-        hipLaunchKernelGGL((march_pass<WW, PP>), dim3(blocks), dim3(256), 0, ctx->stream, table, a);    \
+        hipLaunchKernelGGL((march_pass<WW, PP>), dim3(blocks * turns), dim3(256), 0, ctx->stream, table, a); \
     } while (0)
         if (W == 16) {
             if (precision == LYAP_PREC_PLAIN) LYAP_LAUNCH(16, LYAP_PREC_PLAIN);
@@ -718,7 +731,7 @@ int launch_refine(lyap_ctx *ctx, unsigned n_views, uint32_t subs, uint64_t rays,
     ra.counts = b.refine_counts;
     ra.eval_counter = (unsigned long long *)b.counters;
     const uint32_t cus = ctx->num_cus > 0 ? (uint32_t)ctx->num_cus : 256u;
-    const uint32_t blocks = cus * 8u;
+    const uint32_t blocks = cus * (many ? kManyRefine : kFewRefine);
 #define LYAP_LAUNCH(WW, PP, MM)                                                                     \
     do {                                                                                            \
         if (many)                                                                                   \
