@@ -442,8 +442,8 @@ def bench_batch(lyap, timer, ctx, n_views):
 
 def bench_mixed(lyap, timer, ctx):
     """The 64-view batch and eight 128^3 volume blocks of the precision
-    workload's parameters (the configured FP64 rule) in one persistent launch
-    sequence, against the views' batch followed by the volumes' own kernels."""
+    workload's parameters (the configured FP64 rule) in one call, against the
+    views' batch followed by the volumes' own kernels."""
     from tests import workloads as W
     from tests.gpu_util import RenderBuffers, device_lights, empty
     views, lights, n_lights = W.batch_views(64, seed=4)

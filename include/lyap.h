@@ -294,7 +294,7 @@ int lyap_timing_collect(lyap_ctx *ctx, double *kernel_ms, uint64_t *launches);
 int lyap_last_evals(lyap_ctx *ctx, uint64_t *count);
 
 /* ------------------------------------------------------------------------ */
-/* Batched views: many cameras in one persistent launch                      */
+/* Batched views: many cameras in one launch sequence                        */
 /* ------------------------------------------------------------------------ */
 
 typedef struct LyapView {
@@ -312,7 +312,8 @@ typedef struct LyapView {
     uint32_t reserved;
 } LyapView;
 
-/* Launch shape of the persistent kernels (the reference's fixed 16x16 and
+/* Launch shape of the persistent kernels; asking for one keeps a batch out of
+ * the march passes (the reference's fixed 16x16 and
  * 8x8x8 blocks, lyap_interactive.cu:64-66 and lyap_calculate.cu:19-24, are
  * what it replaces). Zero fields are filled from the autotuner's choice
  * (lyap_autotune, lyap_autotune_batch) or built-in defaults. */
@@ -328,8 +329,8 @@ typedef struct LyapTuning {
                                   which have no claims */
 } LyapTuning;
 
-/* Renders n_views views in one persistent launch fed by a device work queue
- * of ray tiles. Views may differ in size, camera, parameters and sequence. */
+/* Renders n_views views in one launch sequence (see LYAP_SCHEDULE_BATCHED).
+ * Views may differ in size, camera, parameters and sequence. */
 int lyap_render_batch(lyap_ctx *ctx, const LyapView *views, unsigned n_views,
                       const LyapRenderMode *mode, const LyapTuning *tuning);
 

@@ -572,7 +572,7 @@ class Context:
 
     def run_batch(self, views, blocks, mode: Optional[RenderMode] = None,
                   vol_mode: Optional[VolumeMode] = None, tuning: Optional[Tuning] = None):
-        """Views and volume blocks in one persistent launch sequence (lyap_run_batch)."""
+        """Views and volume blocks in one call (lyap_run_batch)."""
         va = (View * max(len(views), 1))(*views)
         ba = (VolumeBlock * max(len(blocks), 1))(*blocks)
         rc = self.lib.lyap_run_batch(self.h, va, len(views), ba, len(blocks),
