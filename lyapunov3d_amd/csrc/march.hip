@@ -582,20 +582,28 @@ void refine_rays(const ViewDesc *__restrict__ views, RefineArgs a)
 
 /* Pass sequences, "lanes per ray x rounds" and 0 rounds for the last one.
  * Below kManyRays a launch's time is its chain of passes and refinement trips:
- * it takes few passes, samples ahead, and two refining lanes per ray. From
- * there on the chip is full whatever the lanes, and a sample taken past a
- * ray's end costs what a needed one does: one lane per ray for as long as
- * enough rays march, in passes short enough that the lanes of ended rays do
- * not idle long, and one refining lane. Both sides, few / many, in us per
- * frame: 256x256 265 / 335, 512x512 320 / 371, 1024x1024 796 / 864, 1448x1448
- * 1499 / 1464, 2048x2048 2900 / 2584; 64 frames of 512x512 48700 / 38600. The
- * march kernel in levels takes 355, 509 and 1765 us for the first three and
- * 51900 for the 64. */
+ * it takes few passes, samples ahead, and two refining lanes per ray. Below
+ * kSmallRays, where a pass raises its lanes per ray far above the minimum, its
+ * first passes take one or two rounds, as most rays end within those samples;
+ * above it, where they do not, four rounds save listing the rays again. Short
+ * / long first passes, in us per frame: 74x370 plain 270 / 300, 170x278 plain
+ * 309 / 342, 256x256 product 251 / 256, plain 380 / 408, FP64 377 / 414,
+ * 512x512 307 / 293, 768x768 544 / 530, 1024x1024 853 / 793.
+ * From kManyRays on the chip is full whatever the lanes, and a sample taken
+ * past a ray's end costs what a needed one does: one lane per ray for as long
+ * as enough rays march, in passes short enough that the lanes of ended rays do
+ * not idle long, and one refining lane. Long first passes / one lane: 256x256
+ * 265 / 335, 512x512 320 / 371, 1024x1024 796 / 864, 1448x1448 1499 / 1464,
+ * 2048x2048 2900 / 2584; 64 frames of 512x512 48700 / 38600. The march kernel
+ * in levels takes 355, 509 and 1765 us for the first three and 51900 for the
+ * 64. */
+constexpr uint64_t kSmallRays = 200000;
 constexpr uint64_t kManyRays = 1800000;
 /* Blocks: a pass of many rays gets kManyTurns grids' worth, and the refinement
  * several per slot, so that a slot whose blocks had cheap rays takes another
  * one: 64 frames of 512x512 take 41.4 ms with one grid each and 37.3 so. */
 constexpr uint32_t kManyTurns = 4, kFewRefine = 16, kManyRefine = 64;
+const char *const kSmallPasses = "2x1,2x2,4x2,8x2,16x4,32x4,64x0";
 const char *const kFewPasses = "2x4,4x4,8x4,16x4,32x4,64x4,64x0";
 const char *const kManyPasses = "1x4,1x4,1x8,1x8,1x16,1x16,2x16,2x16,4x16,8x16,16x8,64x0";
 
@@ -611,7 +619,7 @@ MarchPlan march_plan(unsigned n_views, uint64_t rays)
     if (n_views > 64u) return mp;      /* a wave holds the counts of 64 lists */
     mp.subs = n_views <= 8u ? 8u : 64u / n_views;
     static const char *env = std::getenv("LYAP_MARCH_PASSES");
-    const char *c = env ? env : rays < kManyRays ? kFewPasses : kManyPasses;
+    const char *c = env ? env : rays < kSmallRays ? kSmallPasses : rays < kManyRays ? kFewPasses : kManyPasses;
     if (c[0] == '0' && c[1] == 0) return mp;
     while (*c && mp.n < kMaxPasses) {
         char *e = nullptr;

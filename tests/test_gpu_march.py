@@ -49,14 +49,14 @@ def frame(ctx, w, h, seq, prec, sched, **fields):
 # one ray, ragged edges; each kind of step between passes (near and far
 # steps, steps by the length in the box, jitter); marches of many samples, also
 # past the length whose index and offset share a record's word; the two sides
-# of the launch size that changes the passes and the refining lanes (1.8
-# million rays) with ragged rows
+# of the launch sizes that change the passes (200,000 rays) and the refining
+# lanes as well (1.8 million), with ragged rows
 @pytest.mark.parametrize("prec", [lyap.PREC_PLAIN, lyap.PREC_PRODUCT, lyap.PREC_FP64])
 @pytest.mark.parametrize("w,h,fields", [
     (1, 1, {}), (70, 33, {}), (63, 5, {"nearMultiplier": 3.0}), (40, 41, {"stepMethod": 1, "nearMultiplier": 2.0}),
     (40, 41, {"stepMethod": 0}), (24, 17, {"jitter": 0.5}), (24, 17, {"jitter": 0.5, "stepMethod": 1}),
     (64, 64, {"depth": 2000.0}), (4, 3, {"depth": 80000.0, "stepMethod": 1}), (4, 3, {"depth": 80000.0, "stepMethod": 0}),
-    (1344, 1336, {"depth": 16.0}), (1345, 1344, {"depth": 16.0, "nearMultiplier": 2.0})])
+    (440, 440, {"depth": 48.0}), (449, 448, {"depth": 48.0}), (1344, 1336, {"depth": 16.0}), (1345, 1344, {"depth": 16.0, "nearMultiplier": 2.0})])
 def test_bytes_equal_the_other_schedules(ctx, w, h, fields, prec):
     got = frame(ctx, w, h, "BCABA", prec, lyap.SCHEDULE_BATCHED, **fields)
     for sched in (lyap.SCHEDULE_LEVELS, lyap.SCHEDULE_DIRECT):
