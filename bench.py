@@ -866,7 +866,7 @@ def main():
             "traffic": traffic,
             "traffic_source": traffic_src,
             "flop_per_lambda_eval": flops(prm),
-            "kernel": ("ray_start + march_pass x 7 + refine_rays" if round(launches_per_frame) == 9
+            "kernel": ("march_start + march_pass x 7 + refine_rays" if round(launches_per_frame) == 9
                        else "render_persistent (4 levels) + refine_rays"),
             "launches_per_frame": launches_per_frame,
             "avg_launch_us": launch_ms * 1e3,
