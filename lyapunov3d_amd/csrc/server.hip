@@ -6,10 +6,8 @@
  * runs the launches. Every slot owns a context of its own (stream, launch
  * buffers, counters), so launches of different slots overlap on the device
  * and a launch that is finishing its long rays shares the CUs with the next
- * one. A mixed slot runs its views' ray tiles and its volumes' voxel tiles
- * in one persistent launch (lyap_run_batch's path: the first launch's work
- * queue deals the ray tiles and then the voxel tiles, so the waves whose rays
- * end take voxels). With LYAP_SERVER_SEPARATE_VOLUMES (or when the volume
+ * one. A mixed slot runs its views in one launch sequence and then its
+ * volumes' slabs in the volume kernels (lyap_run_batch's path). With LYAP_SERVER_SEPARATE_VOLUMES (or when the volume
  * precision differs from the views') render slots take views only and
  * volume slots run slabs in the volume kernels.
  *
